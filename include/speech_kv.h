@@ -80,13 +80,17 @@ enum skv_attn_flags {
                                       order, so the launch need not rank them itself */
 };
 
+/* Activations of skv_decode_linear. */
+enum skv_activation { SKV_ACT_NONE = 0, SKV_ACT_GELU = 1 /* x/2 (1 + erf(x / sqrt 2)) */ };
+
 enum skv_status {
   SKV_OK = 0,
   SKV_EINVAL = -1,     /* bad size / null pointer / unsupported head_dim */
   SKV_EDTYPE = -2,     /* unknown dtype code */
   SKV_EALIGN = -3,     /* pointer or stride not 16-byte aligned */
   SKV_EWORKSPACE = -4, /* workspace missing or smaller than skv_attention_workspace_bytes */
-  SKV_EUNSUPPORTED = -5 /* skv_linear: no workspace-free hipBLASLt algorithm for the shape */
+  SKV_EUNSUPPORTED = -5 /* skv_linear: no workspace-free hipBLASLt algorithm for the shape;
+                           skv_decode_linear: not a decode projection's shape or layout */
 };
 
 /* Library version string, e.g. "speechkv 0.3.0 gfx950 src:0123456789abcdef"; the
@@ -358,6 +362,47 @@ SKV_API int skv_codebook_embed_sum(const int64_t* codes, int64_t codes_stride, i
  */
 SKV_API int skv_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, void* y,
                        int64_t ldy, int32_t m, int32_t n, int32_t k, int32_t dtype, void* stream);
+
+/*
+ * skv_decode_linear — a decode batch's projection on the matrix cores, with its activation.
+ *   y[r*ldy + j] = act(sum_i x[r*ldx + i] * w[j*ldw + i] (+ bias[j])) for r < m, j < n, i < k:
+ *   row-major x [m, k], w [n, k], y [m, n]; products and sums in fp32 (the activation too), rounded
+ *   to dtype once. act: SKV_ACT_NONE or SKV_ACT_GELU. bias: [n] in dtype, or NULL.
+ *   A row's bits do not depend on m or on the other rows.
+ * SKV_EUNSUPPORTED (nothing launched; the caller runs another GEMM): a batch that a large-matrix GEMM
+ * serves better (m above 128, unless m <= 512 and m * n is small), rows of less than 512 bytes or not of
+ * whole 16-byte vectors, n not a multiple of 4, an unaligned pointer or stride, x or w past 2 GiB, or rows
+ * past 4 KiB, which skv_decode_linear_splits(k, dtype) > 1 says: those are summed from partials (below).
+ * Replaces the nn.Linear (and GELU) calls of the decoder step, speech_serving/models.py:127-207.
+ */
+SKV_API int skv_decode_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, int32_t act,
+                              void* y, int64_t ldy, int32_t m, int32_t n, int32_t k, int32_t dtype, void* stream);
+
+/*
+ * Workgroups that share the contraction of one output of a projection over k elements of dtype (1: none do,
+ * skv_decode_linear writes the result itself). 0 for a bad argument.
+ */
+SKV_API int32_t skv_decode_linear_splits(int32_t k, int32_t dtype);
+
+/*
+ * skv_decode_linear_partials — the fp32 partial products of x w^T: part[s][r][j], s < skv_decode_linear_splits(k, dtype),
+ * their sum over s being the product. Shapes, layouts and SKV_EUNSUPPORTED as in skv_decode_linear; part_floats is
+ * the size of part (SKV_EWORKSPACE when it is less than splits * m * n).
+ */
+SKV_API int skv_decode_linear_partials(const void* x, int64_t ldx, const void* w, int64_t ldw, float* part,
+                                       int64_t part_floats, int32_t m, int32_t n, int32_t k, int32_t dtype,
+                                       void* stream);
+
+/*
+ * skv_reduce_add_layernorm — skv_add_layernorm of x and the projection whose partials are given:
+ *   sum  = x + (part[0] + part[1] + ... + part[splits-1] + bias), summed in fp32 and rounded to dtype once
+ *          (x NULL: the projection itself; sum may be x; bias NULL: none)
+ *   norm = LayerNorm(sum) * gamma + beta as skv_add_layernorm (gamma, beta and norm NULL: only sum is stored)
+ *   part : [splits][rows][hidden] fp32 (skv_decode_linear_partials); sizes and alignment as skv_add_layernorm.
+ */
+SKV_API int skv_reduce_add_layernorm(const float* part, int32_t splits, const void* bias, const void* x, int64_t ldx,
+                                     const void* gamma, const void* beta, float eps, void* sum, int64_t lds, void* norm,
+                                     int64_t ldn, int32_t rows, int32_t hidden, int32_t dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -29,6 +29,35 @@ __device__ __forceinline__ void store_stream(uint4* p, const uint4& v) {
   __builtin_nontemporal_store(u32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(p));
 }
 
+// Matrix-core operands and results: 8 16-bit contraction elements per lane in, 4 fp32 rows of one column out.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int DT>
+__device__ __forceinline__ f32x4 mfma_16x16x32(const uint4& a, const uint4& b, const f32x4& c) {
+  if constexpr (DT == SKV_BF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                   0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
+                                                  0, 0);
+  }
+}
+
+// Two fp32 values rounded to the dtype (to nearest even) and packed, first value in the
+// low half: v_cvt_pk_bf16_f32 / v_cvt_pk_f16 style conversions, no branches.
+template <int DT>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  const f32x2 f = {a, b};
+  if constexpr (DT == SKV_BF16) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf162v));
+  } else {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, half2v));
+  }
+}
+
 // Element traits: EPL = elements carried by one 16-byte lane load.
 template <int DT> struct Elt;
 template <> struct Elt<SKV_F32> { static constexpr int EPL = 4; };
@@ -50,6 +79,24 @@ __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
   _Float16 ha = (_Float16)a, hb = (_Float16)b;
   uint16_t ua = __builtin_bit_cast(uint16_t, ha), ub = __builtin_bit_cast(uint16_t, hb);
   return (uint32_t)ua | ((uint32_t)ub << 16);
+}
+
+// The fp32 values of a word of two 16-bit elements.
+template <int DT>
+__device__ __forceinline__ float lo16(uint32_t w) {
+  if constexpr (DT == SKV_BF16) {
+    return bf16_lo(w);
+  } else {
+    return (float)__builtin_bit_cast(half2v, w).x;
+  }
+}
+template <int DT>
+__device__ __forceinline__ float hi16(uint32_t w) {
+  if constexpr (DT == SKV_BF16) {
+    return bf16_hi(w);
+  } else {
+    return (float)__builtin_bit_cast(half2v, w).y;
+  }
 }
 
 // Sum over the EPL lane elements of q*k in fp32. fp16/bf16 use the packed

@@ -551,14 +551,7 @@ void launch_argmax(int vecs, int32_t rows, hipStream_t s, const char* logits, in
   }
 }
 
-// ---------------------------------------------------------------------------
-// Residual add + LayerNorm of a decode batch (the pre-LN transformer's
-// `x = x + f(x); h = norm(x)`): sum = x + y rounded to the tensor type, as the
-// separate add would store it; norm = (sum - mean) / sqrt(var + eps) * gamma +
-// beta over the row with fp32 statistics (population variance, two passes over
-// registers), as torch.nn.LayerNorm computes it. One wave per row holds the row
-// in registers: VPL 16-byte vectors per lane.
-// ---------------------------------------------------------------------------
+// The fp32 values of one 16-byte vector.
 template <int DT> __device__ __forceinline__ void unpack16(const uint4& v, float* f);
 template <> __device__ __forceinline__ void unpack16<SKV_F32>(const uint4& v, float* f) {
   f[0] = __uint_as_float(v.x), f[1] = __uint_as_float(v.y), f[2] = __uint_as_float(v.z), f[3] = __uint_as_float(v.w);
@@ -578,99 +571,6 @@ template <> __device__ __forceinline__ void unpack16<SKV_BF16>(const uint4& v, f
   for (int i = 0; i < 4; ++i) {
     f[2 * i] = bf16_lo(w[i]);
     f[2 * i + 1] = bf16_hi(w[i]);
-  }
-}
-
-struct AddNormParams {
-  const uint4* x;
-  const uint4* y;  // NULL: no add
-  const uint4* gamma;
-  const uint4* beta;
-  uint4* sum;      // NULL: sum not stored
-  uint4* norm;
-  int64_t ldx, ldy, lds, ldn;  // row strides in 16-byte vectors
-  int32_t rows, vecs;          // vectors per row
-  float eps, inv_n;
-};
-
-template <int DT, int VPL>
-__global__ __launch_bounds__(256) void add_layernorm_kernel(AddNormParams p) {
-  constexpr int EPL = Elt<DT>::EPL;
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= p.rows) return;  // uniform over the wave
-  float v[VPL][EPL];
-  uint4 raw[VPL], gv[VPL], bv[VPL];
-  // Every load up front (x, y, gamma, beta): one memory round trip per row.
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int c = lane + 64 * j;
-    const bool in = c < p.vecs;
-    raw[j] = in ? p.x[row * p.ldx + c] : make_uint4(0u, 0u, 0u, 0u);
-    gv[j] = in ? p.gamma[c] : make_uint4(0u, 0u, 0u, 0u);
-    bv[j] = in ? p.beta[c] : make_uint4(0u, 0u, 0u, 0u);
-  }
-  if (p.y) {
-    uint4 ry[VPL];
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      const int c = lane + 64 * j;
-      ry[j] = c < p.vecs ? p.y[row * p.ldy + c] : make_uint4(0u, 0u, 0u, 0u);
-    }
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      float a[EPL], b[EPL];
-      unpack16<DT>(raw[j], a);
-      unpack16<DT>(ry[j], b);
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) a[e] += b[e];
-      raw[j] = pack16<DT>(a);  // rounded to the tensor type, like the stored sum
-      const int c = lane + 64 * j;
-      if (p.sum && c < p.vecs) p.sum[row * p.lds + c] = raw[j];
-    }
-  }
-  float s = 0.f;
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    unpack16<DT>(raw[j], v[j]);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) s += v[j][e];
-  }
-  const float mean = group_sum<64>(s) * p.inv_n;
-  float q = 0.f;
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    if (lane + 64 * j < p.vecs) {
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        const float d = v[j][e] - mean;
-        q = fmaf(d, d, q);
-      }
-    }
-  }
-  const float rstd = rsqrtf(group_sum<64>(q) * p.inv_n + p.eps);
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int c = lane + 64 * j;
-    if (c >= p.vecs) continue;
-    float g[EPL], b[EPL], o[EPL];
-    unpack16<DT>(gv[j], g);
-    unpack16<DT>(bv[j], b);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) o[e] = (v[j][e] - mean) * rstd * g[e] + b[e];
-    p.norm[row * p.ldn + c] = pack16<DT>(o);
-  }
-}
-
-template <int DT>
-void launch_add_layernorm(const AddNormParams& p, int vpl, hipStream_t s) {
-  const dim3 grid((uint32_t)cdiv(p.rows, 4));
-  switch (vpl) {
-    case 1: hipLaunchKernelGGL((add_layernorm_kernel<DT, 1>), grid, dim3(256), 0, s, p); break;
-    case 2: hipLaunchKernelGGL((add_layernorm_kernel<DT, 2>), grid, dim3(256), 0, s, p); break;
-    case 3: hipLaunchKernelGGL((add_layernorm_kernel<DT, 3>), grid, dim3(256), 0, s, p); break;
-    case 4: hipLaunchKernelGGL((add_layernorm_kernel<DT, 4>), grid, dim3(256), 0, s, p); break;
-    default: hipLaunchKernelGGL((add_layernorm_kernel<DT, 8>), grid, dim3(256), 0, s, p); break;
   }
 }
 
@@ -1542,50 +1442,6 @@ __global__ __launch_bounds__(256) void merge_kernel(AttnParams p) {
 // The waves merge through LDS; a split row writes per-query partials that
 // merge_kernel combines.
 // ---------------------------------------------------------------------------
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <int DT>
-__device__ __forceinline__ f32x4 mfma_16x16x32(const uint4& a, const uint4& b, const f32x4& c) {
-  if constexpr (DT == SKV_BF16) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
-                                                  0, 0);
-  }
-}
-
-// Two fp32 values rounded to the dtype (to nearest even) and packed, first value in the
-// low half: v_cvt_pk_bf16_f32 / v_cvt_pk_f16 style conversions, no branches.
-template <int DT>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  const f32x2 f = {a, b};
-  if constexpr (DT == SKV_BF16) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf162v));
-  } else {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, half2v));
-  }
-}
-template <int DT>
-__device__ __forceinline__ float lo16(uint32_t w) {
-  if constexpr (DT == SKV_BF16) {
-    return bf16_lo(w);
-  } else {
-    return (float)__builtin_bit_cast(half2v, w).x;
-  }
-}
-template <int DT>
-__device__ __forceinline__ float hi16(uint32_t w) {
-  if constexpr (DT == SKV_BF16) {
-    return bf16_hi(w);
-  } else {
-    return (float)__builtin_bit_cast(half2v, w).y;
-  }
-}
-
 // V^T operand of one 16-dim block straight from row-major LDS rows with the gfx950
 // transpose load ds_read_b64_tr_b16. Within each 16-lane group, element j of lane i's
 // result is element i % 4 of the 8-byte chunk addressed by lane 4j + i / 4 of the group
@@ -2666,46 +2522,6 @@ int skv_argmax(const void* logits, int64_t row_stride, int32_t rows, int32_t voc
       break;
   }
   return check_launch("skv_argmax");
-}
-
-int skv_add_layernorm(const void* x, int64_t ldx, const void* y, int64_t ldy, const void* gamma, const void* beta,
-                      float eps, void* sum, int64_t lds, void* norm, int64_t ldn, int32_t rows, int32_t hidden,
-                      int32_t dtype, void* stream) {
-  const int eb = elt_bytes(dtype);
-  if (eb == 0) return fail(SKV_EDTYPE, "skv_add_layernorm: unknown dtype %d", dtype);
-  const int epl = 16 / eb;
-  if (rows < 0 || hidden <= 0 || hidden % epl || hidden > 64 * 8 * epl)
-    return fail(SKV_EINVAL, "skv_add_layernorm: hidden %d must be a multiple of %d and at most %d (rows=%d)", hidden,
-                epl, 64 * 8 * epl, rows);
-  if (rows == 0) return SKV_OK;
-  if (!x || !gamma || !beta || !norm) return fail(SKV_EINVAL, "skv_add_layernorm: null pointer argument");
-  if (!aligned16(x) || !aligned16(gamma) || !aligned16(beta) || !aligned16(norm) || (y && !aligned16(y)) ||
-      (sum && !aligned16(sum)) || ldx % epl || ldy % epl || lds % epl || ldn % epl)
-    return fail(SKV_EALIGN, "skv_add_layernorm: rows must be 16-byte aligned");
-  if (!(eps >= 0.f)) return fail(SKV_EINVAL, "skv_add_layernorm: eps must be >= 0");
-  AddNormParams p{};
-  p.x = (const uint4*)x;
-  p.y = (const uint4*)y;
-  p.gamma = (const uint4*)gamma;
-  p.beta = (const uint4*)beta;
-  p.sum = y ? (uint4*)sum : nullptr;
-  p.norm = (uint4*)norm;
-  p.ldx = ldx / epl;
-  p.ldy = ldy / epl;
-  p.lds = lds / epl;
-  p.ldn = ldn / epl;
-  p.rows = rows;
-  p.vecs = hidden / epl;
-  p.eps = eps;
-  p.inv_n = 1.f / (float)hidden;
-  const int vpl = (int)cdiv(p.vecs, 64);
-  hipStream_t s = (hipStream_t)stream;
-  switch (dtype) {
-    case SKV_F32: launch_add_layernorm<SKV_F32>(p, vpl, s); break;
-    case SKV_F16: launch_add_layernorm<SKV_F16>(p, vpl, s); break;
-    default: launch_add_layernorm<SKV_BF16>(p, vpl, s); break;
-  }
-  return check_launch("skv_add_layernorm");
 }
 
 int skv_codebook_embed_sum(const int64_t* codes, int64_t codes_stride, int32_t rows, const void* const* tables,

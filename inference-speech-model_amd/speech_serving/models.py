@@ -33,7 +33,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass
-from typing import Any, List, Optional, Sequence, Tuple
+from typing import Any, List, Optional, Sequence, Tuple, Union
 
 import torch
 import torch.nn as nn
@@ -234,35 +234,68 @@ def _hooked(mod: nn.Module) -> bool:
                 nn.modules.module._global_forward_pre_hooks)
 
 
+def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+            gelu: bool = False) -> torch.Tensor:
+    """x @ weight.T (+ bias), then the erf GELU when gelu: a decode batch in one skv_decode_linear launch, other
+    shapes through skv_linear (a hipBLASLt plan cached per shape) and torch's GELU."""
+    y = native.decode_linear(x, weight, bias, gelu)
+    if y is None:
+        y = native.linear(x, weight, bias)
+        if gelu:
+            y = F.gelu(y)
+    return y
+
+
 def proj(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """mod(x). A plain nn.Linear without hooks on a GPU tensor runs as one skv_linear call (a hipBLASLt plan
-    cached per shape: the algorithm and bits of torch's linear without its per-call descriptor set-up and
-    heuristic); any other module, or one with hooks, is called as usual."""
+    """mod(x). A plain nn.Linear without hooks on a GPU tensor runs as one native projection (_linear); any other
+    module, or one with hooks, is called as usual."""
     if x.is_cuda and type(mod) is nn.Linear and not _hooked(mod):
-        return native.linear(x, mod.weight, mod.bias)
+        return _linear(x, mod.weight, mod.bias)
     return mod(x)
 
 
-def mlp(seq: nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """seq(x) for the layers' Linear-GELU-Linear MLP, its projections through proj() (other modules and
-    hooked ones are called as usual)."""
+def _mlp(seq: nn.Module, x: torch.Tensor) -> Union[torch.Tensor, native.Partials]:
+    """seq(x) for the layers' Linear-GELU-Linear MLP, its projections native (other modules and hooked ones are
+    called as usual); the result as Partials when its last projection's contraction is split."""
     if x.is_cuda and type(seq) is nn.Sequential and not _hooked(seq):
         parts = tuple(seq._modules.values())
         if len(parts) == 3 and type(parts[1]) is nn.GELU and not _hooked(parts[1]):
-            return proj(parts[2], F.gelu(proj(parts[0], x), approximate=parts[1].approximate))
+            fc1, act, fc2 = parts
+            if act.approximate == "none" and type(fc1) is nn.Linear and not _hooked(fc1):
+                h = _linear(x, fc1.weight, fc1.bias, gelu=True)
+            else:
+                h = F.gelu(proj(fc1, x), approximate=act.approximate)
+            if type(fc2) is nn.Linear and not _hooked(fc2):
+                y = native.decode_partials(h, fc2.weight, fc2.bias)
+                if y is not None:
+                    return y
+            return proj(fc2, h)
     return seq(x)
 
 
-def add_norm(x: torch.Tensor, y: Optional[torch.Tensor], norm: nn.LayerNorm) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(s, norm(s)) for s = x + y (s = x when y is None): one skv_add_layernorm launch
-    on the GPU, the same two torch ops elsewhere."""
+def _tensor(y: Union[torch.Tensor, native.Partials]) -> torch.Tensor:
+    return y.tensor() if isinstance(y, native.Partials) else y
+
+
+def mlp(seq: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """seq(x) for the layers' Linear-GELU-Linear MLP (see _mlp)."""
+    return _tensor(_mlp(seq, x))
+
+
+def add_norm(x: torch.Tensor, y: Union[torch.Tensor, native.Partials, None],
+             norm: nn.LayerNorm) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(s, norm(s)) for s = x + y (s = x when y is None): one native launch on the GPU (which also sums
+    the Partials of a split projection), the same two torch ops elsewhere."""
     if x.is_cuda and norm.elementwise_affine and not _hooked(norm):
         bias = norm.bias
         if bias is not None:
-            got = native.add_layernorm(x, y, norm.weight, bias, norm.eps, fallback=True)
+            if isinstance(y, native.Partials):
+                got = native.reduce_add_layernorm(y, x, norm.weight, bias, norm.eps)
+            else:
+                got = native.add_layernorm(x, y, norm.weight, bias, norm.eps, fallback=True)
             if got is not None:
                 return got
-    s = x if y is None else x + y
+    s = x if y is None else x + _tensor(y)
     return s, norm(s)
 
 
@@ -333,7 +366,7 @@ class DecoderLayer(nn.Module):
         """q, k, v [B, S, H, D] from the already normalised input h."""
         b, s, _ = h.shape
         hd = self.num_heads * self.head_dim
-        qkv = native.linear(h, self.qkv_weight()) if h.is_cuda else F.linear(h, self.qkv_weight())
+        qkv = _linear(h, self.qkv_weight()) if h.is_cuda else F.linear(h, self.qkv_weight())
         shape = (b, s, self.num_heads, self.head_dim)
         return qkv[..., :hd].view(shape), qkv[..., hd:2 * hd].view(shape), qkv[..., 2 * hd:].view(shape)
 
@@ -352,6 +385,12 @@ class DecoderLayer(nn.Module):
         (pending: the previous layer's MLP output, not yet added). Returns (x, mlp
         output) with the MLP output left for the next layer (or the final norm) to
         add, so every residual add shares a launch with the LayerNorm that follows it."""
+        x, y = self._step_paged(x, layer, kv, cross, pending)
+        return x, _tensor(y)
+
+    def _step_paged(self, x: torch.Tensor, layer: int, kv: PagedKV, cross: Optional[CrossKV],
+                    pending: Union[torch.Tensor, native.Partials, None]):
+        """forward_paged with the MLP output in and out as the projection left it (_mlp)."""
         b, s, _ = x.shape
         hd = self.num_heads * self.head_dim
         x, h = add_norm(x, pending, self.norm1)
@@ -369,7 +408,7 @@ class DecoderLayer(nn.Module):
             x, h = add_norm(x, proj(self.cross_attn_out, c.view(b, s, hd)), self.norm3)
         else:
             x, h = add_norm(x, a, self.norm2)
-        return x, mlp(self.mlp, h)
+        return x, _mlp(self.mlp, h)
 
     # -- contiguous API of the reference (models.py:110-208) ---------------------
     def forward(self, x: torch.Tensor, past_key_values: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
@@ -422,6 +461,16 @@ class DecoderLayer(nn.Module):
             c = native.dense_attention(self._cross_q(x), ck, cv, clens, te, self.scale)
             x = x + proj(self.cross_attn_out, c.reshape(b, s, hd))
         return self._finish(x, used), new_past, new_cross
+
+
+def _layer_step(layer: nn.Module, x: torch.Tensor, index: int, kv: PagedKV, cross: Optional[CrossKV],
+                pending: Union[torch.Tensor, native.Partials, None]):
+    """layer.forward_paged, its MLP output handed on as the projection left it; a layer whose forward_paged is
+    overridden is called through it, with tensors."""
+    if getattr(type(layer), "forward_paged", None) is DecoderLayer.forward_paged and \
+            "forward_paged" not in layer.__dict__:
+        return layer._step_paged(x, index, kv, cross, pending)
+    return layer.forward_paged(x, index, kv, cross, None if pending is None else _tensor(pending))
 
 
 # ---------------------------------------------------------------------------
@@ -507,12 +556,12 @@ class WhisperClassSpeechEncoderDecoderModel(nn.Module):
         x = self._embed(input_ids)
         pending = None
         for l, layer in enumerate(self.decoder_layers):
-            x, pending = layer.forward_paged(x, l, kv, cross, pending)
-        if last_only:
-            x = x[:, -1]
-            pending = None if pending is None else pending[:, -1]
+            x, pending = _layer_step(layer, x, l, kv, cross, pending)
+        if last_only and x.shape[1] > 1:
+            x = x[:, -1:]
+            pending = None if pending is None else _tensor(pending)[:, -1:]
         _, h = add_norm(x, pending, self.decoder_norm)
-        return proj(self.lm_head, h)
+        return proj(self.lm_head, h[:, 0] if last_only else h)
 
     # -- decode step, reference signature (models.py:369-423) ----------------------------
     def decode_step(self, input_ids: torch.Tensor, past_key_values: Optional[Any] = None,
@@ -704,7 +753,7 @@ class MultiCodebookHeads(nn.Module):
         """[B, S, hidden] -> logits [B, S, K, V]."""
         b, s, _ = hidden_states.shape
         w = self.fused_weight()
-        y = native.linear(hidden_states, w) if hidden_states.is_cuda else F.linear(hidden_states, w)
+        y = _linear(hidden_states, w) if hidden_states.is_cuda else F.linear(hidden_states, w)
         return y.view(b, s, self.num_codebooks, self.vocab_size)
 
 
@@ -791,10 +840,10 @@ class StreamingMultiCodebookTTSModel(nn.Module):
         x = self.embeddings(input_codebooks)
         pending = None
         for l, layer in enumerate(self.layers):
-            x, pending = layer.forward_paged(x, l, kv, None, pending)
-        if last_only:
+            x, pending = _layer_step(layer, x, l, kv, None, pending)
+        if last_only and x.shape[1] > 1:
             x = x[:, -1:]
-            pending = None if pending is None else pending[:, -1:]
+            pending = None if pending is None else _tensor(pending)[:, -1:]
         _, h = add_norm(x, pending, self.norm)
         logits = self.heads(h)
         return logits[:, 0] if last_only else logits

@@ -11,6 +11,8 @@ Functions:
     dense_attention(q, k, v, lens, max_len, scale, ...)
     argmax(logits, ...), copy_cross_kv(...), add_layernorm(...), codebook_embed_sum(...)
     linear(x, weight, bias)   (hipBLASLt with a plan cached per shape)
+    decode_linear(x, weight, bias, gelu), decode_partials(x, weight, bias), reduce_add_layernorm(...)
+                              (a decode batch's projections on the matrix cores)
 """
 from __future__ import annotations
 
@@ -60,8 +62,17 @@ SIGNATURES = {
     "skv_codebook_embed_sum": (_c_int, [_c_p, _c_i64, _c_i32, _c_p, _c_i32, _c_i32, _c_i32, _c_p, _c_i64, _c_i32,
                                         _c_p]),
     "skv_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_p]),
+    "skv_decode_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_i64, _c_i32, _c_i32, _c_i32,
+                                   _c_i32, _c_p]),
+    "skv_decode_linear_splits": (_c_i32, [_c_i32, _c_i32]),
+    "skv_decode_linear_partials": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
+                                            _c_p]),
+    "skv_reduce_add_layernorm": (_c_int, [_c_p, _c_i32, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_f, _c_p, _c_i64, _c_p,
+                                          _c_i64, _c_i32, _c_i32, _c_i32, _c_p]),
 }
-SKV_EUNSUPPORTED = -5  # skv_linear: no workspace-free hipBLASLt algorithm for the shape
+SKV_EUNSUPPORTED = -5  # skv_linear, skv_decode_linear: not a shape or layout the call takes
+SKV_ACT_NONE, SKV_ACT_GELU = 0, 1
+MAX_DECODE_ROWS = 512  # most rows skv_decode_linear takes (kMaxRows of the library)
 MAX_CODEBOOKS = 16  # kMaxCodebooks of the library
 
 
@@ -612,6 +623,108 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         return torch.nn.functional.linear(x, weight, bias)
     _check(rc, "skv_linear")
     return y
+
+
+def _proj_operands(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]):
+    """(x as [m, k] rows, m, n, k, dtype code) of a decode projection, or None when the batch, the types or the
+    layouts are not those skv_decode_linear takes (its own checks decide about sizes and alignment)."""
+    k = x.shape[-1]
+    code = _DTYPE_CODE.get(x.dtype)
+    if code is None or not x.is_cuda or not weight.is_cuda or weight.dtype != x.dtype or weight.dim() != 2 or \
+            weight.shape[1] != k or weight.stride(1) != 1 or x.numel() > MAX_DECODE_ROWS * k or k == 0:
+        return None
+    n = weight.shape[0]
+    if bias is not None and (bias.dtype != x.dtype or bias.dim() != 1 or bias.shape[0] != n or bias.stride(0) != 1
+                             or not bias.is_cuda):
+        return None
+    x2 = x.reshape(-1, k)
+    if x2.stride(1) != 1 or (x2.shape[0] > 1 and x2.stride(0) < k):
+        return None
+    return x2, x2.shape[0], n, k, code
+
+
+def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                  gelu: bool = False) -> Optional[torch.Tensor]:
+    """act(x @ weight.T (+ bias)) of a decode batch (or a short prompt batch) in one launch on the matrix cores, summed
+    in fp32 and rounded once; gelu applies the erf GELU to the fp32 result. None for a call skv_decode_linear does
+    not take (the caller runs linear()). Reference: speech_serving/models.py:127-207."""
+    ops = _proj_operands(x, weight, bias)
+    if ops is None:
+        return None
+    x2, m, n, k, code = ops
+    y = torch.empty(x.shape[:-1] + (n,), dtype=x.dtype, device=x.device)
+    rc = lib().skv_decode_linear(x2.data_ptr(), x2.stride(0) if m > 1 else k, weight.data_ptr(),
+                                 weight.stride(0) if n > 1 else k, _ptr(bias), SKV_ACT_GELU if gelu else SKV_ACT_NONE,
+                                 y.data_ptr(), n, m, n, k, code, _stream(x.device))
+    if rc == SKV_EUNSUPPORTED:
+        return None
+    _check(rc, "skv_decode_linear")
+    return y
+
+
+class Partials:
+    """A projection whose contraction several workgroups share: fp32 partial products [splits, rows, n] that the next
+    residual add + LayerNorm sums (reduce_add_layernorm), or tensor() when the result itself is wanted."""
+
+    __slots__ = ("part", "bias", "shape", "dtype")
+
+    def __init__(self, part: torch.Tensor, bias: Optional[torch.Tensor], shape: torch.Size, dtype: torch.dtype):
+        self.part, self.bias, self.shape, self.dtype = part, bias, shape, dtype
+
+    def tensor(self) -> torch.Tensor:
+        return reduce_add_layernorm(self, None, None, None, 0.0)[0]
+
+
+@functools.lru_cache(maxsize=256)
+def _decode_splits(k: int, code: int) -> int:
+    return int(lib().skv_decode_linear_splits(k, code))
+
+
+def decode_partials(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[Partials]:
+    """x @ weight.T (+ bias) as Partials when the projection's contraction is split, else None (a call that
+    decode_linear or linear takes)."""
+    ops = _proj_operands(x, weight, bias)
+    if ops is None:
+        return None
+    x2, m, n, k, code = ops
+    splits = _decode_splits(k, code)
+    epl = 16 // x.element_size()
+    # a row's sum is one reduce_add_layernorm row: its sizes and alignment
+    if splits <= 1 or m == 0 or n % epl or n > 512 * epl or (bias is not None and bias.data_ptr() % 16):
+        return None
+    part = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+    rc = lib().skv_decode_linear_partials(x2.data_ptr(), x2.stride(0) if m > 1 else k, weight.data_ptr(),
+                                          weight.stride(0) if n > 1 else k, part.data_ptr(), part.numel(), m, n, k,
+                                          code, _stream(x.device))
+    if rc == SKV_EUNSUPPORTED:
+        return None
+    _check(rc, "skv_decode_linear_partials")
+    return Partials(part, bias, x.shape[:-1] + (n,), x.dtype)
+
+
+def reduce_add_layernorm(p: Partials, x: Optional[torch.Tensor], weight: Optional[torch.Tensor],
+                         bias: Optional[torch.Tensor], eps: float) -> Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]]:
+    """(s, LayerNorm(s)) with s = x + the projection p, summed in fp32 and rounded once (x None: the projection;
+    weight None: s alone). None for an x or LayerNorm that add_layernorm does not take either."""
+    splits, rows, h = p.part.shape
+    x2 = None
+    if x is not None:
+        got = _layernorm_rows(x, x if weight is None else weight)
+        if got is None or x.dtype != p.dtype or x.shape != p.shape:
+            return None
+        x2 = got[0]
+    if weight is not None and (weight.dtype != p.dtype or not weight.is_contiguous() or weight.numel() != h or
+                               weight.data_ptr() % 16 or bias.dtype != p.dtype or not bias.is_contiguous() or
+                               bias.numel() != h or bias.data_ptr() % 16):
+        return None
+    s = torch.empty(p.shape, dtype=p.dtype, device=p.part.device)
+    norm = None if weight is None else torch.empty(p.shape, dtype=p.dtype, device=p.part.device)
+    rc = lib().skv_reduce_add_layernorm(p.part.data_ptr(), splits, _ptr(p.bias), _ptr(x2),
+                                        x2.stride(0) if x2 is not None and rows > 1 else h, _ptr(weight),
+                                        None if weight is None else bias.data_ptr(), float(eps), s.data_ptr(), h,
+                                        _ptr(norm), h, rows, h, _DTYPE_CODE[p.dtype], _stream(p.part.device))
+    _check(rc, "skv_reduce_add_layernorm")
+    return s, norm
 
 
 def add_layernorm_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
