@@ -230,10 +230,10 @@ SKV_API int32_t skv_paged_chunk_tokens(int32_t rows, int32_t num_heads, int32_t 
  *              pools at pool[table[pos / block_size], pos % block_size] (the
  *              reference's slot-mapping scatter, phase_aware_scheduler.py:
  *              1004-1010 and :681-690) and attends over them in the same launch.
- * A row with 0 visible keys gets a zero output. Non-causal calls with q_len >= 2 and
- * no fused append (attention over an encoder table), head_dim 64, fp16/bf16 and a
- * power-of-two block size of at least 8 run every 16 queries of a row against one
- * read of its blocks, with both products on the matrix cores; with 64 or more
+ * A row with 0 visible keys gets a zero output. Calls with q_len >= 2 (attention over an
+ * encoder table; prompts of some size, causal and with a fused append), head_dim 64,
+ * fp16/bf16 and a power-of-two block size of at least 8 run every 16 queries of a row
+ * against one read of its blocks, with both products on the matrix cores; with 64 or more
  * queries per row and (row, head, 64-query) workgroups for at least three quarters
  * of the GPU's compute units, every 64 queries share one read of the blocks staged
  * in LDS.
@@ -294,8 +294,8 @@ SKV_API int skv_paged_attention_noalloc(const void* q, int64_t q_stride_b, int64
  *   Row b reads slot slot_ids ? slot_ids[b] : b.
  *   lens  : int32 [B] keys visible to the last query of row b (causal as above).
  * Used for cross-attention over g_cross_kv [S, L, 2, H, T_enc, D] slices and for
- * causal attention over contiguous prompt K/V. Non-causal calls with q_len >= 2
- * (a prompt's cross-attention), head_dim 64 and fp16/bf16 run every 16 queries of
+ * causal attention over contiguous prompt K/V. Calls with q_len >= 2 (a prompt's
+ * cross-attention, larger causal prompts), head_dim 64 and fp16/bf16 run every 16 queries of
  * a row against one read of its K/V, with both products on the matrix cores (every
  * 64 queries, staged in LDS, when rows carry 64 or more queries and the
  * (row, head, 64-query) workgroups cover at least three quarters of the GPU).

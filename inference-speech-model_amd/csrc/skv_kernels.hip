@@ -1416,10 +1416,11 @@ __global__ __launch_bounds__(256) void merge_kernel(AttnParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Multi-query attention over contiguous K/V on the matrix cores (cross-attention
-// of a prompt, q_len >= 2, non-causal, head_dim 64, fp16/bf16).
+// Multi-query attention on the matrix cores (q_len >= 2, head_dim 64, fp16/bf16): the
+// cross-attention of a prompt, attention over encoder blocks, and a prompt's own causal
+// attention with its fused append (PROMPT).
 //
-// One workgroup of kWaves waves owns one (row, head, tile of 16 queries, key
+// One workgroup of WAVES waves owns one (row, head, tile of 16 queries, key
 // chunk): the tile's queries share every K/V load, so K/V are read once per tile
 // instead of once per query. Per 32 keys a wave runs
 //   S^T[32 keys x 16 q] = K . Q^T   4 x v_mfma_f32_16x16x32 (2 key tiles x 2 dim slabs)
@@ -1437,8 +1438,8 @@ __global__ __launch_bounds__(256) void merge_kernel(AttnParams p) {
 // Online softmax per query (base 2), the max over a 32-key step reduced across
 // the 4 lane groups. P enters its product with V in the input dtype: fp16 rounds
 // it once (the row sums then add the rounded values, so the weights stay a convex
-// combination); bf16 adds the product of the rounded remainder, which keeps the
-// weights to ~16 bits.
+// combination); bf16, and prompts in either dtype, add the product of the rounded
+// remainder, which keeps the weights to ~16 bits (fp16 22).
 // The waves merge through LDS; a split row writes per-query partials that
 // merge_kernel combines.
 // ---------------------------------------------------------------------------
@@ -1458,6 +1459,76 @@ __device__ __forceinline__ uint4 vt_operand(const char* row_a, const char* row_b
   return make_uint4(ua.x, ua.y, ub.x, ub.y);
 }
 
+// Prompts (PROMPT variants of the two kernels below): causal queries, and with a fused append the Q
+// newest keys of a row read from the caller's k_new / v_new rows, which the workgroups of the first head
+// of each KV group write into the pool.
+//
+// A key that some queries of a tile see and others do not has weight 0 for the latter, and 0 times an
+// infinite or NaN V is NaN: a tile whose result is not finite is computed again, one query at a time
+// over exactly the keys it sees (query_slow).
+struct PromptRow {
+  int row_len, qlen, max_len, causal;
+  // Keys visible to query qi.
+  __device__ __forceinline__ int visible(int qi) const {
+    int len = row_len - (causal ? qlen - 1 - qi : 0);
+    len = len < 0 ? 0 : len;
+    return len > max_len ? max_len : len;
+  }
+};
+
+// Appends row b's new keys first .. first + count - 1 (counted from new_begin, positions 0 .. end - 1 only) of KV head
+// kvh into the pools, by the whole workgroup: each tile of queries writes the keys of its own tokens.
+__device__ __forceinline__ void append_new_rows(const AttnParams& p, int b, int kvh, const int32_t* tbl, int new_begin,
+                                                int first, int count, int end, int lpt) {
+  const int w0 = max(new_begin + first, 0);
+  const int nw = max(min(end, new_begin + first + count) - w0, 0) * lpt;
+  for (int i = threadIdx.x; i < 2 * nw; i += blockDim.x) {
+    const int kv = i >= nw;
+    const int r = i - kv * nw;
+    const int t = w0 + r / lpt, j = r % lpt;
+    const uint32_t blk = (uint32_t)tbl[t >> p.bs_shift];
+    if (blk < (uint32_t)p.nb) {
+      const int64_t dst = ((int64_t)blk * p.bs + (t & (p.bs - 1))) * p.row_vecs + (int64_t)kvh * lpt + j;
+      const int64_t src = (int64_t)b * p.nsb + (int64_t)(t - new_begin) * p.nsq + (int64_t)kvh * p.nsh + j;
+      const_cast<uint4*>(kv ? p.v : p.k)[dst] = (kv ? p.vn : p.kn)[src];
+    }
+  }
+}
+
+// One query (head_dim 64) by one wave, a dim per lane: keys [t0, t1) one after the other.
+template <int DT, bool PAGED>
+__device__ __forceinline__ void query_slow(const AttnParams& p, int b, int qi, int h, int kvh, int t0, int t1,
+                                                     int new_begin, float& m, float& l, float& acc) {
+  using elt = typename std::conditional<DT == SKV_F16, _Float16, __bf16>::type;
+  const int lane = threadIdx.x & 63;
+  const float q = (float)reinterpret_cast<const elt*>(p.q + (int64_t)b * p.qsb + (int64_t)qi * p.qsq +
+                                                      (int64_t)h * p.qsh)[lane];
+  const int32_t* tbl = PAGED ? p.tables + (int64_t)(p.trows ? p.trows[b] : b) * p.tstride : nullptr;
+  m = kNegInf, l = 0.f, acc = 0.f;
+  for (int t = t0; t < t1; ++t) {
+    const uint4 *kr, *vr;
+    if (PAGED && t >= new_begin) {
+      const int64_t off = (int64_t)b * p.nsb + (int64_t)(t - new_begin) * p.nsq + (int64_t)kvh * p.nsh;
+      kr = p.kn + off, vr = p.vn + off;
+    } else if (PAGED) {
+      const uint32_t blk = (uint32_t)tbl[t >> p.bs_shift];
+      if (blk >= (uint32_t)p.nb) continue;
+      const int64_t off = ((int64_t)blk * p.bs + (t & (p.bs - 1))) * p.row_vecs + (int64_t)kvh * 8;
+      kr = p.k + off, vr = p.v + off;
+    } else {
+      const int64_t off = (int64_t)(p.slots ? p.slots[b] : b) * p.ss + (int64_t)kvh * p.sh + (int64_t)t * p.st;
+      kr = p.k + off, vr = p.v + off;
+    }
+    const float s = group_sum<64>(q * (float)reinterpret_cast<const elt*>(kr)[lane]) * p.scale_log2;
+    const float mx = fmaxf(m, s);
+    const float ref = mx == kNegInf ? 0.f : mx;
+    const float a = __builtin_amdgcn_exp2f(m - ref), w = __builtin_amdgcn_exp2f(s - ref);
+    l = l * a + w;
+    acc = fmaf(w, (float)reinterpret_cast<const elt*>(vr)[lane], acc * a);
+    m = mx;
+  }
+}
+
 constexpr int kMqQueries = 16;  // queries per tile (the MFMA's N)
 // Lazy rescaling of the matrix-core kernels' online softmax: a wave's reference maximum
 // (and with it the accumulators' scale) moves only when some query's step maximum exceeds it
@@ -1466,23 +1537,24 @@ constexpr int kMqQueries = 16;  // queries per tile (the MFMA's N)
 // query's maximum grows in most steps: rescaling at every growth multiplied the accumulators
 // almost every step.
 constexpr float kLazyMaxLog2 = 8.f;
-static_assert(kWaves == 4, "mq_attention_kernel: each of the 4 waves finalises one 16-dim block");
 
 // 3 waves per SIMD: the register budget that holds the next step's loads in flight without
 // spilling (4 spills and halves the rate; 2 is no faster).
 // PAGED: K/V come from the block pools through the row's table (power-of-two block size of
 // at least 8 keys, so the 8 keys of one load instruction share a block id, read with a
 // scalar load); otherwise from the contiguous [slot, head, T, D] layout.
-template <int DT, bool PAGED>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(3))) void
+template <int DT, bool PAGED, bool PROMPT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3))) void
 mq_attention_kernel(AttnParams p, int32_t qtiles) {
+  static_assert(WAVES == 4 || WAVES == 1, "each wave finalises 4 / WAVES of the 16-dim blocks");
+  constexpr bool kSplitP = DT == SKV_BF16 || PROMPT;  // P as a rounded head plus the rounded remainder
   constexpr int D = 64;
   constexpr int PSTRIDE = D + kPartPad;
-  __shared__ float s_m[kWaves][kMqQueries];
-  __shared__ float s_l[kWaves][kMqQueries];
+  __shared__ float s_m[WAVES][kMqQueries];
+  __shared__ float s_l[WAVES][kMqQueries];
   // Per-wave K/V staging rows during the key loop; the wave merge reuses the space.
-  constexpr int kStageBytes = kWaves * 2 * 32 * (D * 2 + 16);
-  static_assert(kStageBytes >= (int)sizeof(float) * kWaves * kMqQueries * (D + 4), "merge buffer fits the staging");
+  constexpr int kStageBytes = WAVES * 2 * 32 * (D * 2 + 16);
+  static_assert(kStageBytes >= (int)sizeof(float) * WAVES * kMqQueries * (D + 4), "merge buffer fits the staging");
   __shared__ __attribute__((aligned(16))) char s_stage[kStageBytes];
   auto s_acc = reinterpret_cast<float (*)[kMqQueries][D + 4]>(s_stage);
 
@@ -1491,19 +1563,35 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
   const int g = lane >> 4;   // lane group of the MFMA layouts
   const int n = lane & 15;   // query column (result, P^T) / key or dim row (operands)
   const int h = (int)(blockIdx.x % (uint32_t)p.heads);
-  const int qt = (int)(blockIdx.x / (uint32_t)p.heads);
+  int qt = (int)(blockIdx.x / (uint32_t)p.heads);
+  if constexpr (PROMPT) qt = qtiles - 1 - qt;  // the tiles that see the most keys first
   const int b = blockIdx.y;
   const int chunk = blockIdx.z;
   const int kvh = p.group == 1 ? h : h / p.group;
 
   int len = p.lens[b];
+  const PromptRow prow{len, p.qlen, p.max_len, p.causal};
   len = len < 0 ? 0 : (len > p.max_len ? p.max_len : len);
   const int qi = qt * kMqQueries + n;  // this lane's query (result layout)
   const bool q_ok = qi < p.qlen;
+  // Keys this lane's query sees, the least any query of the tile sees, and the first key read from k_new.
+  int my_len = len, min_len = len, new_begin = 0x7fffffff;
+  if constexpr (PROMPT) {
+    if (PAGED && p.kn) {
+      new_begin = len - p.qlen;
+      if (chunk == 0 && h % p.group == 0)
+        append_new_rows(p, b, kvh, p.tables + (int64_t)(p.trows ? p.trows[b] : b) * p.tstride, new_begin,
+                        qt * kMqQueries, kMqQueries, len, D / 8);
+    }
+    len = prow.visible(min(qt * kMqQueries + kMqQueries, p.qlen) - 1);
+    my_len = prow.visible(min(qi, p.qlen - 1));
+    min_len = prow.visible(qt * kMqQueries);
+  }
   if (len == 0) {
-    if (chunk == 0 && wave < 4 && q_ok) {  // zero output: lane writes dims 16*wave + 4g .. +4
+    if (chunk == 0 && q_ok) {  // zero output: lane writes dims 16*db + 4g .. +4
       uint2* o = reinterpret_cast<uint2*>(p.o + (int64_t)b * p.osb + (int64_t)qi * p.osq + (int64_t)h * p.osh);
-      o[(16 * wave + 4 * g) / 4] = make_uint2(0u, 0u);
+#pragma unroll
+      for (int db = 4 / WAVES * wave; db < 4 / WAVES * (wave + 1); ++db) o[(16 * db + 4 * g) / 4] = make_uint2(0u, 0u);
     }
     return;
   }
@@ -1539,16 +1627,22 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
       __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kb), (short)0, (int)p.kv_bytes, kBufWord3);
   const __amdgpu_buffer_rsrc_t vres =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vb), (short)0, (int)p.kv_bytes, kBufWord3);
+  // The chunk's keys [t_begin, pool_end) come from the pool or the contiguous rows, [pool_end, t_end) from k_new / v_new.
+  const int pool_end = PROMPT ? max(t_begin, min(new_begin, t_end)) : t_end;
+  const int pool_steps = (pool_end - t_begin + 31) >> 5;
+  const int steps = PROMPT ? pool_steps + ((t_end - pool_end + 31) >> 5) : pool_steps;
+  const int64_t noff = (PAGED && PROMPT && p.kn) ? (int64_t)b * p.nsb + (int64_t)kvh * p.nsh : 0;
+  const uint32_t new_bytes = (uint32_t)(((p.qlen - 1) * p.nsq + D / 8) * 16);
   // Byte offset of key `key` (its row's column base added), out of range past t_end or
   // behind an invalid block id. key0 is the wave-uniform first key of a load instruction;
   // blk_ok reports (wave-uniformly) whether those 8 keys have a valid block.
   auto key_offset = [&](int key0, int key, bool& blk_ok) -> uint32_t {
     if constexpr (PAGED) {
       // Clamped to the last key so the table index stays inside the row (which covers max_len).
-      const uint32_t k0 = (uint32_t)__builtin_amdgcn_readfirstlane(min(key0, t_end - 1));
+      const uint32_t k0 = (uint32_t)__builtin_amdgcn_readfirstlane(min(key0, pool_end - 1));
       const uint32_t blk = trow[k0 >> p.bs_shift];  // wave-uniform: a scalar load
       blk_ok = blk < (uint32_t)p.nb;
-      return key < t_end && blk_ok
+      return key < pool_end && blk_ok
                  ? (blk * (uint32_t)p.bs + ((uint32_t)key & ((uint32_t)p.bs - 1u))) * row_bytes + col_base
                  : kBufOutOfRange;
     } else {
@@ -1577,8 +1671,32 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
   char* lds_v = lds_k + STEP * kRowPad;
   const int nat_row = lane >> 3, nat_col = (lane & 7) * 16;  // key row / byte column of a load
   // Returns the step's valid-key mask (bit j: key base + j lies in a valid block).
-  auto load_step = [&](int base, uint4 (&kr)[4], uint4 (&vr)[4]) -> uint32_t {
+  // First key of a step.
+  auto step_base = [&](int step) -> int {
+    return PROMPT && step >= pool_steps ? pool_end + (step - pool_steps) * STEP : t_begin + step * STEP;
+  };
+  auto load_step = [&](int step, uint4 (&kr)[4], uint4 (&vr)[4]) -> uint32_t {
+    const int base = step_base(step);
     uint32_t off[4], mask = 0u;
+    if constexpr (PAGED && PROMPT) {
+      if (step >= pool_steps) {  // wave-uniform
+        const __amdgpu_buffer_rsrc_t nkres = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint4*>(p.kn + noff), (short)0, (int)new_bytes, kBufWord3);
+        const __amdgpu_buffer_rsrc_t nvres = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint4*>(p.vn + noff), (short)0, (int)new_bytes, kBufWord3);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = base + 8 * i + nat_row;
+          off[i] = key < t_end ? (uint32_t)(key - new_begin) * (uint32_t)p.nsq * 16u + (uint32_t)nat_col : kBufOutOfRange;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          kr[i] = load_buf(nkres, off[i]);
+          vr[i] = load_buf(nvres, off[i]);
+        }
+        return 0xffffffffu;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       bool blk_ok;
@@ -1593,7 +1711,9 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
     }
     return mask;
   };
-  auto compute_step = [&](int base, const uint4 (&kr)[4], const uint4 (&vr)[4], uint32_t mask) {
+  auto compute_step = [&](int step, const uint4 (&kr)[4], const uint4 (&vr)[4], uint32_t mask) {
+    const int base = step_base(step);
+    const int end = PROMPT && step < pool_steps ? pool_end : t_end;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       *reinterpret_cast<uint4*>(lds_k + (8 * i + nat_row) * kRowPad + nat_col) = kr[i];
@@ -1623,13 +1743,15 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) sv[4 * t + i] = sc[t][i] * p.scale_log2;
-    if (base + STEP > t_end || (PAGED && mask != 0xffffffffu)) {  // wave-uniform: a chunk's last step or an invalid block
+    // Wave-uniform: a chunk's last step, an invalid block, or a key that some query does not see
+    if (base + STEP > min(end, min_len) || (PAGED && mask != 0xffffffffu)) {
+      const int lim = min(end, my_len);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int kk = 16 * t + 4 * g + i;
-          const bool ok = base + kk < t_end && (!PAGED || ((mask >> kk) & 1u));
+          const bool ok = base + kk < lim && (!PAGED || ((mask >> kk) & 1u));
           sv[4 * t + i] = ok ? sv[4 * t + i] : kNegInf;
         }
     }
@@ -1662,7 +1784,7 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
       const float p1 = __builtin_amdgcn_exp2f(sv[2 * k + 1] - ref);
       const uint32_t w = pack2<DT>(p0, p1);
       pw[k] = w;
-      if constexpr (DT == SKV_BF16) {
+      if constexpr (kSplitP) {
         pr[k] = pack2<DT>(p0 - lo16<DT>(w), p1 - hi16<DT>(w));
         l += p0 + p1;
       } else {
@@ -1674,23 +1796,22 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
       acc[db] = mfma_16x16x32<DT>(vt[db], pt, acc[db]);
-      if constexpr (DT == SKV_BF16) acc[db] = mfma_16x16x32<DT>(vt[db], prt, acc[db]);
+      if constexpr (kSplitP) acc[db] = mfma_16x16x32<DT>(vt[db], prt, acc[db]);
     }
   };
   // Software pipeline: the next step's loads are in flight while this step computes.
-  const int stride = kWaves * STEP;
-  int s0 = t_begin + wave * STEP;
+  int s0 = wave;
   uint4 ka[4], va[4], kb2[4], vb2[4];
   uint32_t ma = 0u, mb = 0u;
-  if (s0 < t_end) ma = load_step(s0, ka, va);
-  while (s0 < t_end) {
-    const int s1 = s0 + stride;
-    if (s1 < t_end) mb = load_step(s1, kb2, vb2);
+  if (s0 < steps) ma = load_step(s0, ka, va);
+  while (s0 < steps) {
+    const int s1 = s0 + WAVES;
+    if (s1 < steps) mb = load_step(s1, kb2, vb2);
     __builtin_amdgcn_sched_barrier(0);
     compute_step(s0, ka, va, ma);
-    if (s1 >= t_end) break;
-    const int s2 = s1 + stride;
-    if (s2 < t_end) ma = load_step(s2, ka, va);
+    if (s1 >= steps) break;
+    const int s2 = s1 + WAVES;
+    if (s2 < steps) ma = load_step(s2, ka, va);
     __builtin_amdgcn_sched_barrier(0);
     compute_step(s1, kb2, vb2, mb);
     s0 = s2;
@@ -1699,49 +1820,89 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
   l += xor_lane<16>(l);
   l += xor_lane<32>(l);
 
-  // Merge the waves: wave w then finalises dim block w for the 16 queries. The merge buffer
+  // Merge the waves: wave w then finalises dim block w for the 16 queries (one wave: all four). The merge buffer
   // overlaps the other waves' staging rows, so every wave leaves its key loop first.
-  __syncthreads();
-  if (g == 0) {
-    s_m[wave][n] = m;
-    s_l[wave][n] = l;
+  constexpr int kBlocks = 4 / WAVES;  // dim blocks a wave finalises
+  float M = m, L = l;
+  f32x4 A[kBlocks];
+  if constexpr (WAVES == 1) {
+#pragma unroll
+    for (int db = 0; db < 4; ++db) A[db] = acc[db];
+  } else {
+    __syncthreads();
+    if (g == 0) {
+      s_m[wave][n] = m;
+      s_l[wave][n] = l;
+    }
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s_acc[wave][n][16 * db + 4 * g + i] = acc[db][i];
+    __syncthreads();
+    M = kNegInf;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) M = fmaxf(M, s_m[w][n]);
+    const float mref = M == kNegInf ? 0.f : M;
+    L = 0.f;
+    A[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float e = __builtin_amdgcn_exp2f(s_m[w][n] - mref);
+      L += e * s_l[w][n];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) A[0][i] += e * s_acc[w][n][16 * wave + 4 * g + i];
+    }
   }
+  if constexpr (PROMPT) {
+    // A sum that is not finite: the tile again, one query at a time (4 queries per wave).
+    float sum = L;
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s_acc[wave][n][16 * db + 4 * g + i] = acc[db][i];
-  __syncthreads();
-  if (wave >= 4) return;
-  float M = kNegInf;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) M = fmaxf(M, s_m[w][n]);
-  const float mref = M == kNegInf ? 0.f : M;
-  float L = 0.f, A[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    const float e = __builtin_amdgcn_exp2f(s_m[w][n] - mref);
-    L += e * s_l[w][n];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) A[i] += e * s_acc[w][n][16 * wave + 4 * g + i];
+    for (int db = 0; db < kBlocks; ++db) sum += fabsf(A[db][0]) + fabsf(A[db][1]) + fabsf(A[db][2]) + fabsf(A[db][3]);
+    const bool bad = q_ok && !(sum < __builtin_huge_valf());
+    if (__syncthreads_or(bad)) {
+      for (int i = 0; i < kMqQueries / WAVES; ++i) {
+        const int qs = qt * kMqQueries + wave * (kMqQueries / WAVES) + i;
+        if (qs >= p.qlen) break;
+        const int vis = prow.visible(qs);
+        if (chunk > 0 && t_begin >= vis) continue;
+        float m1, l1, a1;
+        query_slow<DT, PAGED>(p, b, qs, h, kvh, t_begin, min(t_end, vis), new_begin, m1, l1, a1);
+        if (p.nchunk_max == 1 || vis <= p.chunk) {
+          reinterpret_cast<uint16_t*>(p.o + (int64_t)b * p.osb + (int64_t)qs * p.osq + (int64_t)h * p.osh)[lane] =
+              (uint16_t)pack2<DT>(l1 > 0.f ? a1 * (1.f / l1) : (l1 == 0.f ? 0.f : l1), 0.f);
+        } else {
+          float* rec = p.part + ((((int64_t)b * p.qlen + qs) * p.heads + h) * p.nchunk_max + chunk) * PSTRIDE;
+          rec[kPartPad + lane] = a1;
+          if (lane == 0) *reinterpret_cast<float2*>(rec) = make_float2(m1, l1);
+        }
+      }
+      return;
+    }
   }
   if (!q_ok) return;
-  const int d0 = 16 * wave + 4 * g;
-  if (nchunks == 1) {
+  // A query whose keys fit one chunk gets its output here, the others a partial per chunk of theirs.
+  const bool whole = PROMPT ? p.nchunk_max == 1 || my_len <= p.chunk : nchunks == 1;
+  if (whole) {
+    if (PROMPT && chunk > 0) return;
     const float inv = L > 0.f ? 1.f / L : 0.f;
     uint2* o = reinterpret_cast<uint2*>(p.o + (int64_t)b * p.osb + (int64_t)qi * p.osq + (int64_t)h * p.osh);
-    o[d0 / 4] = make_uint2(pack2<DT>(A[0] * inv, A[1] * inv), pack2<DT>(A[2] * inv, A[3] * inv));
+#pragma unroll
+    for (int db = 0; db < kBlocks; ++db)
+      o[(16 * (wave * kBlocks + db) + 4 * g) / 4] =
+          make_uint2(pack2<DT>(A[db][0] * inv, A[db][1] * inv), pack2<DT>(A[db][2] * inv, A[db][3] * inv));
     return;
   }
   const int64_t rh = ((int64_t)b * p.qlen + qi) * p.heads + h;
   float* rec = p.part + (rh * p.nchunk_max + chunk) * PSTRIDE;
-  *reinterpret_cast<float4*>(rec + kPartPad + d0) = make_float4(A[0], A[1], A[2], A[3]);
+#pragma unroll
+  for (int db = 0; db < kBlocks; ++db)
+    *reinterpret_cast<f32x4*>(rec + kPartPad + 16 * (wave * kBlocks + db) + 4 * g) = A[db];
   if (wave == 0 && g == 0) *reinterpret_cast<float2*>(rec) = make_float2(M, L);
 }
 
 // ---------------------------------------------------------------------------
 // Multi-query attention with many queries per row (encoder attention over a
-// table of encoder blocks, q_len = T; long prompts), fp16/bf16, head_dim 64,
-// non-causal: one workgroup owns 64 queries of one (row, head), 16 per wave, and
+// table of encoder blocks, q_len = T; long prompts), fp16/bf16, head_dim 64: one workgroup owns 64 queries of one (row, head), 16 per wave, and
 // walks the row's keys in 64-key steps staged in LDS, so K/V are read once per
 // 64 queries (mq_attention_kernel reads them once per 16). The workgroup is two
 // parts of 4 waves: part 0 takes the first half of the steps, part 1 the second,
@@ -1759,11 +1920,12 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
 constexpr int kMqtQueries = 64;  // queries per workgroup, 16 per wave of a part
 constexpr int kMqtParts = 2;     // key halves per workgroup
 
-template <int DT, bool PAGED>
+template <int DT, bool PAGED, bool PROMPT>
 __global__ __launch_bounds__(64 * kWaves * kMqtParts) __attribute__((amdgpu_waves_per_eu(4))) void
 mqt_attention_kernel(AttnParams p) {
   static_assert(kWaves * kMqQueries == kMqtQueries, "mqt_attention_kernel: 16 queries per wave");
   static_assert(kMqtParts == 2, "mqt_attention_kernel: the end-of-kernel merge is written for two parts");
+  constexpr bool kSplitP = DT == SKV_BF16 || PROMPT;  // P as a rounded head plus the rounded remainder
   constexpr int D = 64;
   constexpr int STEP = 32;                       // keys per compute half-step
   constexpr int LSTEP = 64;                      // keys per staged step, 16 per wave
@@ -1779,14 +1941,31 @@ mqt_attention_kernel(AttnParams p) {
   const int g = lane >> 4;  // lane group of the MFMA layouts
   const int n = lane & 15;  // query column (result, P^T) / key or dim row (operands)
   const int h = (int)(blockIdx.x % (uint32_t)p.heads);
-  const int qg = (int)(blockIdx.x / (uint32_t)p.heads);
+  int qg = (int)(blockIdx.x / (uint32_t)p.heads);
+  if constexpr (PROMPT) qg = (int)(gridDim.x / (uint32_t)p.heads) - 1 - qg;  // the most keys first
   const int b = blockIdx.y;
   const int kvh = p.group == 1 ? h : h / p.group;
 
   int len = p.lens[b];
+  const PromptRow prow{len, p.qlen, p.max_len, p.causal};
   len = len < 0 ? 0 : (len > p.max_len ? p.max_len : len);
-  const int qi = qg * kMqtQueries + wave * kMqQueries + n;  // this lane's query (result layout)
+  const int q0 = qg * kMqtQueries + wave * kMqQueries;  // the wave's first query
+  const int qi = q0 + n;                                // this lane's query (result layout)
   const bool q_ok = qi < p.qlen;
+  // Keys this lane's query sees, the least and the most any query of the wave sees, and the first key read from k_new.
+  int my_len = len, min_len = len, max_len = len, new_begin = 0x7fffffff;
+  if constexpr (PROMPT) {
+    if (PAGED && p.kn) {
+      new_begin = len - p.qlen;
+      if (h % p.group == 0)
+        append_new_rows(p, b, kvh, p.tables + (int64_t)(p.trows ? p.trows[b] : b) * p.tstride, new_begin,
+                        qg * kMqtQueries, kMqtQueries, len, D / 8);
+    }
+    len = prow.visible(min(qg * kMqtQueries + kMqtQueries, p.qlen) - 1);
+    my_len = prow.visible(min(qi, p.qlen - 1));
+    min_len = prow.visible(min(q0, p.qlen - 1));
+    max_len = prow.visible(min(q0 + kMqQueries, p.qlen) - 1);
+  }
   if (len == 0) {  // uniform over the workgroup: zero output
     if (q_ok && part == 0) {
       uint2* o = reinterpret_cast<uint2*>(p.o + (int64_t)b * p.osb + (int64_t)qi * p.osq + (int64_t)h * p.osh);
@@ -1828,16 +2007,27 @@ mqt_attention_kernel(AttnParams p) {
   // read of the table row; the steps' presence bits then depend on len only.
   bool row_ok = true;
   if constexpr (PAGED) {
-    const int nblk = (len + p.bs - 1) >> p.bs_shift;
+    const int nblk = (max(0, min(len, new_begin)) + p.bs - 1) >> p.bs_shift;
     bool bad = false;
     for (int e = lane; e < nblk; e += 64) bad |= trow[e] >= (uint32_t)p.nb;
     row_ok = __builtin_amdgcn_ballot_w64(bad) == 0;
   }
 
   // This part's steps: [st0, st0 + nsteps) of the row's ceil(len / 64), keys below lim.
-  const int nsteps = ((len + LSTEP - 1) / LSTEP + kMqtParts - 1) / kMqtParts;
+  // With a fused append the row's steps are those of its pool keys [0, pool_end), then those of the new keys.
+  const int pool_end = PROMPT ? max(0, min(len, new_begin)) : len;
+  const int pool_steps = (pool_end + LSTEP - 1) / LSTEP;
+  const int all_steps = PROMPT ? pool_steps + (len - pool_end + LSTEP - 1) / LSTEP : pool_steps;
+  const int nsteps = (all_steps + kMqtParts - 1) / kMqtParts;
   const int st0 = part * nsteps;
-  const int lim = min(len, (st0 + nsteps) * LSTEP);
+  const int st_lim = min(all_steps, st0 + nsteps);
+  const int lim = min(pool_end, st_lim * LSTEP);
+  const int64_t noff = (PAGED && PROMPT && p.kn) ? (int64_t)b * p.nsb + (int64_t)kvh * p.nsh : 0;
+  const uint32_t new_bytes = (uint32_t)(((p.qlen - 1) * p.nsq + D / 8) * 16);
+  // First key of a step.
+  auto step_base = [&](int st) -> int {
+    return PROMPT && st >= pool_steps ? pool_end + (st - pool_steps) * LSTEP : st * LSTEP;
+  };
 
   // Issues step st's loads for this wave (keys st*64 + 16*wave + 8r + (lane >> 3) for
   // r = 0, 1, byte column 16 * (lane & 7); at or past lim, or behind an invalid block,
@@ -1848,13 +2038,32 @@ mqt_attention_kernel(AttnParams p) {
   // wave's own two, and on a row with an invalid id the step's eight, in one batch.
   const int nat_row = lane >> 3, nat_col = (lane & 7) * 16;
   auto issue = [&](int st, uint4 (&kr)[2], uint4 (&vr)[2]) -> uint64_t {
-    const int base = st * LSTEP;
-    uint64_t bits = base + LSTEP <= len ? ~0ull : (base < len ? (1ull << (len - base)) - 1ull : 0ull);
+    const int base = step_base(st);
+    const int end = PROMPT && st < pool_steps ? pool_end : len;
+    uint64_t bits = base + LSTEP <= end ? ~0ull : (base < end ? (1ull << (end - base)) - 1ull : 0ull);
+    if constexpr (PAGED && PROMPT) {
+      if (st >= pool_steps) {  // wave-uniform: keys of k_new / v_new
+        const __amdgpu_buffer_rsrc_t nkres = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint4*>(p.kn + noff), (short)0, (int)new_bytes, kBufWord3);
+        const __amdgpu_buffer_rsrc_t nvres = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint4*>(p.vn + noff), (short)0, (int)new_bytes, kBufWord3);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const int key = base + 16 * wave + 8 * r + nat_row;
+          const uint32_t off = key < len && st < st_lim
+                                   ? (uint32_t)(key - new_begin) * (uint32_t)p.nsq * 16u + (uint32_t)nat_col
+                                   : kBufOutOfRange;
+          kr[r] = load_buf(nkres, off);
+          vr[r] = load_buf(nvres, off);
+        }
+        return bits;
+      }
+    }
     if constexpr (PAGED) {
       if (!row_ok) {
         uint32_t blk[8];
 #pragma unroll
-        for (int gi = 0; gi < 8; ++gi) blk[gi] = trow[(uint32_t)min(base + 8 * gi, len - 1) >> p.bs_shift];
+        for (int gi = 0; gi < 8; ++gi) blk[gi] = trow[(uint32_t)min(base + 8 * gi, pool_end - 1) >> p.bs_shift];
 #pragma unroll
         for (int gi = 0; gi < 8; ++gi)
           if (blk[gi] >= (uint32_t)p.nb) bits &= ~(0xffull << (8 * gi));
@@ -1866,7 +2075,7 @@ mqt_attention_kernel(AttnParams p) {
       const int key = key0 + nat_row;
       uint32_t off;
       if constexpr (PAGED) {
-        const uint32_t own = trow[(uint32_t)min(key0, len - 1) >> p.bs_shift];
+        const uint32_t own = trow[(uint32_t)min(key0, pool_end - 1) >> p.bs_shift];
         off = key < lim && own < (uint32_t)p.nb
                   ? (own * (uint32_t)p.bs + ((uint32_t)key & ((uint32_t)p.bs - 1u))) * row_bytes + col_base +
                         (uint32_t)nat_col
@@ -1902,7 +2111,7 @@ mqt_attention_kernel(AttnParams p) {
   // fp16 sums P on the matrix cores: a product with an operand of ones gives every lane
   // its query's sum over the step's 32 keys (the rounded weights, as the PV product
   // uses them). bf16 sums the unrounded weights on the VALU: its P is two operands.
-  constexpr bool kOnesSum = DT == SKV_F16;
+  constexpr bool kOnesSum = !kSplitP;
   f32x4 l4 = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint4 ones = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);
 
@@ -1918,7 +2127,8 @@ mqt_attention_kernel(AttnParams p) {
     }
   };
   // Softmax and PV products of one half; keys whose bit is clear score -inf.
-  auto compute = [&](int buf, int half, const f32x4 (&sc)[2], uint32_t bits) __attribute__((always_inline)) {
+  auto compute = [&](int buf, int half, const f32x4 (&sc)[2], uint32_t bits, int base) __attribute__((always_inline)) {
+    if (PROMPT && base >= max_len) return;  // wave-uniform: no query of the wave sees these keys
     const char* lds_v = s_tile[buf] + LSTEP * kRowPad + half * STEP * kRowPad;
     uint4 vt[4];
     {
@@ -1934,12 +2144,15 @@ mqt_attention_kernel(AttnParams p) {
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) sv[4 * t + i] = sc[t][i];
-    if (bits != 0xffffffffu) {  // wave-uniform: a row's last step or an invalid block
+    // Wave-uniform: a row's last step, an invalid block, or a key that some query does not see
+    if (bits != 0xffffffffu || (PROMPT && base + STEP > min_len)) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          sv[4 * t + i] = ((bits >> (16 * t + 4 * g + i)) & 1u) ? sv[4 * t + i] : kNegInf;
+        for (int i = 0; i < 4; ++i) {
+          const int kk = 16 * t + 4 * g + i;
+          sv[4 * t + i] = ((bits >> kk) & 1u) && (!PROMPT || base + kk < my_len) ? sv[4 * t + i] : kNegInf;
+        }
     }
     float mx = kNegInf;
 #pragma unroll
@@ -1972,7 +2185,7 @@ mqt_attention_kernel(AttnParams p) {
       const float p1 = __builtin_amdgcn_exp2f(fmaf(sv[2 * k + 1], p.scale_log2, -ref));
       const uint32_t w = pack2<DT>(p0, p1);
       pw[k] = w;
-      if constexpr (DT == SKV_BF16) {
+      if constexpr (kSplitP) {
         pr[k] = pack2<DT>(p0 - lo16<DT>(w), p1 - hi16<DT>(w));
         l += p0 + p1;
       }
@@ -1982,7 +2195,7 @@ mqt_attention_kernel(AttnParams p) {
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
       acc[db] = mfma_16x16x32<DT>(vt[db], pt, acc[db]);
-      if constexpr (DT == SKV_BF16) acc[db] = mfma_16x16x32<DT>(vt[db], prt, acc[db]);
+      if constexpr (kSplitP) acc[db] = mfma_16x16x32<DT>(vt[db], prt, acc[db]);
     }
     if constexpr (kOnesSum) l4 = mfma_16x16x32<DT>(ones, pt, l4);
   };
@@ -2008,8 +2221,9 @@ mqt_attention_kernel(AttnParams p) {
     f32x4 sc0[2], sc1[2];
     scores(st & 1, 0, sc0);
     scores(st & 1, 1, sc1);  // issued before the first half's softmax, so the two overlap
-    compute(st & 1, 0, sc0, (uint32_t)bits);
-    compute(st & 1, 1, sc1, (uint32_t)(bits >> 32));  // a half with no key changes nothing
+    const int base = PROMPT ? step_base(st0 + st) : 0;
+    compute(st & 1, 0, sc0, (uint32_t)bits, base);
+    compute(st & 1, 1, sc1, (uint32_t)(bits >> 32), base + STEP);  // a half with no key changes nothing
     lds_barrier();
   };
   for (int st = 0; st < nsteps; st += 2) {
@@ -2037,7 +2251,7 @@ mqt_attention_kernel(AttnParams p) {
       for (int i = 0; i < 4; ++i) xs[128 + (4 * db + i) * 64 + lane] = acc[db][i];
   }
   lds_barrier();
-  if (part == 1 || !q_ok) return;
+  if (part == 1 || (!PROMPT && !q_ok)) return;
   {
     const float m1 = xs[lane], l1 = xs[64 + lane];
     const float mm = fmaxf(m, m1);
@@ -2048,6 +2262,22 @@ mqt_attention_kernel(AttnParams p) {
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[db][i] = a0 * acc[db][i] + a1 * xs[128 + (4 * db + i) * 64 + lane];
+  }
+  if constexpr (PROMPT) {
+    // A sum that is not finite: the wave's queries again, one at a time.
+    float sum = l;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) sum += fabsf(acc[db][0]) + fabsf(acc[db][1]) + fabsf(acc[db][2]) + fabsf(acc[db][3]);
+    if (__builtin_amdgcn_ballot_w64(q_ok && !(sum < __builtin_huge_valf())) != 0) {
+      for (int qs = q0; qs < min(q0 + kMqQueries, p.qlen); ++qs) {
+        float m1, l1, a1;
+        query_slow<DT, PAGED>(p, b, qs, h, kvh, 0, prow.visible(qs), new_begin, m1, l1, a1);
+        reinterpret_cast<uint16_t*>(p.o + (int64_t)b * p.osb + (int64_t)qs * p.osq + (int64_t)h * p.osh)[lane] =
+            (uint16_t)pack2<DT>(l1 > 0.f ? a1 * (1.f / l1) : (l1 == 0.f ? 0.f : l1), 0.f);
+      }
+      return;
+    }
+    if (!q_ok) return;
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   uint2* o = reinterpret_cast<uint2*>(p.o + (int64_t)b * p.osb + (int64_t)qi * p.osq + (int64_t)h * p.osh);
@@ -2257,32 +2487,66 @@ int bind_workspace(AttnParams& p, const char* who, int32_t d, void* ws, int64_t 
 
 }  // namespace
 
+// Whether a multi-query launch is a prompt's: causal, or with a fused append.
+bool is_prompt(const AttnParams& p) { return p.causal || p.kn; }
+
+// Prompts of at most this many keys take one wave per (row, head, 16 queries): one or two steps of keys leave nothing
+// for four waves to share, and four times the workgroups are resident (bf16 20 heads, 128 x 4 tokens 6.0 us, with four
+// waves 14.2; 32 x 32 tokens 8.0 / 9.9 us, 8 x 32 6.5 / 5.5 us).
+constexpr int kShortPrompt = 32;
+
+// Whether a prompt's queries go to the matrix-core kernels rather than one workgroup per (query, head): when those
+// would be four per compute unit or more, or have many keys each. Below that the launch is its floor and one
+// query's chain is shorter. Measured (us, one workgroup per query / matrix cores; bf16, fused append):
+//   20 heads: 8 x 4 tokens 4.2 / 4.2, 8 x 16 7.0 / 5.0, 8 x 64 21.6 / 6.2, 8 x 201 84.6 / 16.6, 128 x 4 18.8 / 6.0,
+//   128 x 32 133 / 21, 1 x 32 4.6 / 5.0; 4 heads: 1 x 64 4.7 / 5.5, 1 x 201 10.0 / 5.4, 32 x 8 4.5 / 4.4;
+//   after 200-3000 cached keys, 20 heads: 1 x 2 (400) 5.5 / 8.0, 8 x 2 (200) 6.9 / 7.7, 64 x 2 (200) 23.4 / 20.8,
+//   1 x 16 (3000) 27.5 / 17.8.
+bool prompt_on_mfma(const AttnParams& p) {
+  const int64_t items = (int64_t)p.batch * p.qlen * p.heads, work = items * p.max_len;
+  return (items >= 1024 && (p.qlen >= 4 || p.max_len <= kShortPrompt)) || (p.qlen >= 16 && work >= 40 * 1024) ||
+         work >= 160 * 1024;
+}
+
 // The multi-query matrix-core attention (fp16/bf16, head_dim 64) and, for split rows, the merge.
-template <bool PAGED>
-void launch_mq(int32_t dtype, const AttnParams& p, hipStream_t s) {
+template <int DT, bool PAGED>
+void launch_mq_dt(const AttnParams& p, hipStream_t s) {
   const int32_t qtiles = (int32_t)cdiv(p.qlen, kMqQueries);
   const dim3 grid((uint32_t)(p.heads * qtiles), (uint32_t)p.batch, (uint32_t)p.nchunk_max);
-  if (dtype == SKV_BF16)
-    hipLaunchKernelGGL((mq_attention_kernel<SKV_BF16, PAGED>), grid, dim3(64 * kWaves), 0, s, p, qtiles);
+  if (is_prompt(p) && p.max_len <= kShortPrompt)
+    hipLaunchKernelGGL((mq_attention_kernel<DT, PAGED, true, 1>), grid, dim3(64), 0, s, p, qtiles);
+  else if (is_prompt(p))
+    hipLaunchKernelGGL((mq_attention_kernel<DT, PAGED, true, kWaves>), grid, dim3(64 * kWaves), 0, s, p, qtiles);
   else
-    hipLaunchKernelGGL((mq_attention_kernel<SKV_F16, PAGED>), grid, dim3(64 * kWaves), 0, s, p, qtiles);
+    hipLaunchKernelGGL((mq_attention_kernel<DT, PAGED, false, kWaves>), grid, dim3(64 * kWaves), 0, s, p, qtiles);
   if (p.nchunk_max > 1) {
     const int64_t rh = (int64_t)p.batch * p.qlen * p.heads;
-    if (dtype == SKV_BF16)
-      hipLaunchKernelGGL((merge_kernel<SKV_BF16, 64>), dim3((uint32_t)cdiv(rh, 4)), dim3(256), 0, s, p);
-    else
-      hipLaunchKernelGGL((merge_kernel<SKV_F16, 64>), dim3((uint32_t)cdiv(rh, 4)), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((merge_kernel<DT, 64>), dim3((uint32_t)cdiv(rh, 4)), dim3(256), 0, s, p);
   }
+}
+template <bool PAGED>
+void launch_mq(int32_t dtype, const AttnParams& p, hipStream_t s) {
+  if (dtype == SKV_BF16)
+    launch_mq_dt<SKV_BF16, PAGED>(p, s);
+  else
+    launch_mq_dt<SKV_F16, PAGED>(p, s);
 }
 
 // Many queries per row on the matrix cores: 64 queries per workgroup over all of the row's keys.
+template <int DT, bool PAGED>
+void launch_mqt_dt(const AttnParams& p, hipStream_t s) {
+  const dim3 grid((uint32_t)(p.heads * cdiv(p.qlen, kMqtQueries)), (uint32_t)p.batch, 1u);
+  if (is_prompt(p))
+    hipLaunchKernelGGL((mqt_attention_kernel<DT, PAGED, true>), grid, dim3(64 * kWaves * kMqtParts), 0, s, p);
+  else
+    hipLaunchKernelGGL((mqt_attention_kernel<DT, PAGED, false>), grid, dim3(64 * kWaves * kMqtParts), 0, s, p);
+}
 template <bool PAGED>
 void launch_mqt(int32_t dtype, const AttnParams& p, hipStream_t s) {
-  const dim3 grid((uint32_t)(p.heads * cdiv(p.qlen, kMqtQueries)), (uint32_t)p.batch, 1u);
   if (dtype == SKV_BF16)
-    hipLaunchKernelGGL((mqt_attention_kernel<SKV_BF16, PAGED>), grid, dim3(64 * kWaves * kMqtParts), 0, s, p);
+    launch_mqt_dt<SKV_BF16, PAGED>(p, s);
   else
-    hipLaunchKernelGGL((mqt_attention_kernel<SKV_F16, PAGED>), grid, dim3(64 * kWaves * kMqtParts), 0, s, p);
+    launch_mqt_dt<SKV_F16, PAGED>(p, s);
 }
 
 // Whether the 64-query kernel serves a multi-query launch: enough queries per row,
@@ -2642,13 +2906,15 @@ int paged_attention_impl(const char* who, const void* q, int64_t q_stride_b, int
   p.nb = num_blocks;
   p.row_vecs = (int64_t)num_kv_heads * head_dim / (16 / elt_bytes(dtype));
   p.kv_bytes = (int64_t)num_blocks * block_size * p.row_vecs * 16;
-  // Several non-causal queries per row with no fused append (attention over a whole encoder
-  // table, EncoderAttentionBackend): every 16 queries of a row share one read of its blocks;
-  // the 64-query kernel takes all of a row's keys in one workgroup, so it needs no partials.
-  const bool mq = !p.causal && q_len >= 2 && !k_new && head_dim == 64 && (dtype == SKV_F16 || dtype == SKV_BF16) &&
+  // Several queries per row (attention over a whole encoder table, EncoderAttentionBackend; a prompt with its
+  // fused append): every 16 queries of a row share one read of its blocks; the 64-query kernel takes
+  // all of a row's keys in one workgroup, so it needs no partials. The new keys' rows of one (row, KV head) are
+  // read through a 32-bit descriptor of their own.
+  const bool new_ok = !k_new || (p.nsq >= 0 && (int64_t)(q_len - 1) * p.nsq * 16 + head_dim * 2 <= kBufLimit);
+  const bool mq = q_len >= 2 && new_ok && (!is_prompt(p) || prompt_on_mfma(p)) && head_dim == 64 && (dtype == SKV_F16 || dtype == SKV_BF16) &&
                   p.kv_bytes <= kBufLimit && p.bs_shift >= 3 && batch <= 65535;
   const bool mqt = mq && use_mqt(p);
-  if (mqt) {
+  if (mqt && !is_prompt(p)) {
     p.nchunk_max = 1;
     p.snake = 0;
   }
@@ -2664,6 +2930,8 @@ int paged_attention_impl(const char* who, const void* q, int64_t q_stride_b, int
   }
   if (batch == 0) return SKV_OK;
   if (mq) {
+    // A prompt keeps the workspace it asked for (bind_workspace above), whichever kernel serves it.
+    if (mqt) p.nchunk_max = 1;
     if (mqt)
       launch_mqt<true>(dtype, p, (hipStream_t)stream);
     else
@@ -2733,13 +3001,13 @@ int skv_dense_attention(const void* q, int64_t q_stride_b, int64_t q_stride_q, i
   p.kv_bytes = max_len > 0 ? ((int64_t)(max_len - 1) * (p.st < 0 ? -p.st : p.st) + head_dim / epl) * 16 : 16;
   if (p.st < 0) p.kv_bytes = kBufLimit + 1;  // negative key strides take the 64-bit path
   p.slots = slot_ids;
-  // Several non-causal queries per row (a prompt's cross-attention): one workgroup per
+  // Several queries per row (a prompt's cross-attention, a causal prompt over contiguous K/V): one workgroup per
   // tile of 16 queries reads the row's K/V once and runs both products on the matrix cores;
   // the 64-query kernel takes all of a row's keys in one workgroup (no partials).
-  const bool mq = !p.causal && q_len >= 2 && head_dim == 64 && (dtype == SKV_F16 || dtype == SKV_BF16) &&
+  const bool mq = q_len >= 2 && (!is_prompt(p) || prompt_on_mfma(p)) && head_dim == 64 && (dtype == SKV_F16 || dtype == SKV_BF16) &&
                   p.kv_bytes <= kBufLimit && p.st > 0 && batch <= 65535;
   const bool mqt = mq && use_mqt(p);
-  if (mqt) {
+  if (mqt && !is_prompt(p)) {
     p.nchunk_max = 1;
     p.snake = 0;
   }
@@ -2747,6 +3015,7 @@ int skv_dense_attention(const void* q, int64_t q_stride_b, int64_t q_stride_q, i
   if (rc != SKV_OK) return rc;
   if (batch == 0) return SKV_OK;
   if (mq) {
+    if (mqt) p.nchunk_max = 1;  // a prompt keeps the workspace it asked for, whichever kernel serves it
     if (mqt)
       launch_mqt<false>(dtype, p, (hipStream_t)stream);
     else
