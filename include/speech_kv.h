@@ -372,11 +372,29 @@ SKV_API int skv_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, c
  * SKV_EUNSUPPORTED (nothing launched; the caller runs another GEMM): a batch that a large-matrix GEMM
  * serves better (m above 128, unless m <= 512 and m * n is small), rows of less than 512 bytes or not of
  * whole 16-byte vectors, n not a multiple of 4, an unaligned pointer or stride, x or w past 2 GiB, or rows
- * past 4 KiB, which skv_decode_linear_splits(k, dtype) > 1 says: those are summed from partials (below).
+ * past 6 KiB, which skv_decode_linear_splits(k, dtype) > 1 says: those are summed from partials (below).
  * Replaces the nn.Linear (and GELU) calls of the decoder step, speech_serving/models.py:127-207.
  */
 SKV_API int skv_decode_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, int32_t act,
                               void* y, int64_t ldy, int32_t m, int32_t n, int32_t k, int32_t dtype, void* stream);
+
+/*
+ * skv_decode_linear_fused — skv_decode_linear between a decoder layer's residual adds and LayerNorms:
+ *   y[r*ldy + j] = act(sum_i h[r][i] * w[j*ldw + i] (+ bias[j])) (+ res[r*ldr + j]), the residual added in fp32
+ *     and the sum rounded once; res [m, n] in dtype, or NULL (it may be y).
+ *   h = x, or with x_stats, gamma and beta (all three or none) the LayerNorm of x's rows, rounded to dtype:
+ *     (x - mean) * rsqrt(var + eps) * gamma + beta; gamma, beta [k] in dtype.
+ *   y_stats (or NULL): fp32 [m][n / 16][2], the sum and the sum of squared deviations from their mean of each 16
+ *     consecutive elements of y as stored. x_stats is that of the call that stored x: [m][k / 16][2].
+ * SKV_EUNSUPPORTED besides skv_decode_linear's: y_stats with n, or x_stats with k, not a multiple of 16; x_stats where
+ * a LayerNorm launch ahead of the projection is the faster way (more than 128 rows, rows past 4 KiB, an output of many
+ * tiles); res, bias, gamma, beta or the statistics unaligned.
+ * Reference: the pre-LN residual blocks of speech_serving/models.py:127-207.
+ */
+SKV_API int skv_decode_linear_fused(const void* x, int64_t ldx, const float* x_stats, const void* gamma,
+                                    const void* beta, float eps, const void* w, int64_t ldw, const void* bias,
+                                    int32_t act, const void* res, int64_t ldr, void* y, int64_t ldy, float* y_stats,
+                                    int32_t m, int32_t n, int32_t k, int32_t dtype, void* stream);
 
 /*
  * Workgroups that share the contraction of one output of a projection over k elements of dtype (1: none do,

@@ -10,7 +10,7 @@
 //     are in flight at once, before the first product; nothing is issued past the row;
 //   * loads read whole 128-byte lines (8 lanes per row) and reach the operand layout
 //     through the wave's own padded LDS rows: in operand order every 16 lanes would touch 16 lines;
-//   * rows past 4 KiB (the MLP's second product) are split over workgroups too; the fp32 partials
+//   * rows past 6 KiB (a large MLP's second product) are split over workgroups too; the fp32 partials
 //     are summed by the residual add + LayerNorm that follows, which costs no launch of its own.
 // Workgroups with the same weight tile sit on one XCD (block x is the tile modulo 8), so each XCD's L2 reads
 // its weights from memory once.
@@ -40,6 +40,17 @@ struct ProjEpilogue {
   float* part;       // split: fp32 partials [splits][m][n]; else NULL
   int64_t ldy;       // elements
   int32_t act;       // 1: GELU (erf)
+  const char* res;   // [m, n] added to the fp32 result, at row stride ldr; or NULL
+  int64_t ldr;
+  float2* stats;     // [m, n / 16]: sum and squared deviations of each 16 stored elements; or NULL
+};
+
+// LayerNorm of the x rows before the product (gamma NULL: none).
+struct ProjNorm {
+  const void* gamma;  // [k]
+  const void* beta;
+  const float2* stats;  // [m, k / 16] as ProjEpilogue::stats of the projection that stored x
+  float eps, inv_k;
 };
 
 // One 16 x 16 product step over a 128-byte chunk of 16 weight rows and 16 rows of x, both in LDS
@@ -66,23 +77,99 @@ __device__ __forceinline__ uint4 load_cached(__amdgpu_buffer_rsrc_t r, uint32_t 
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// The elements of a 16-byte vector of x, normalised and rounded to the dtype: (x - mean) * rstd * gamma + beta.
+// st: mean and rstd, for 16-bit rows -mean * rstd and rstd (one operation less; the fp32 rounding it adds is
+// |mean / std| 2^-24 against the 2^-9 or 2^-12 of the result).
 template <int DT>
-__device__ __forceinline__ float load_elt(const void* p, uint32_t i) {
-  if constexpr (DT == SKV_F32) {
-    return static_cast<const float*>(p)[i];
-  } else if constexpr (DT == SKV_F16) {
-    return (float)static_cast<const _Float16*>(p)[i];
-  } else {
-    return bf16_lo(static_cast<const uint16_t*>(p)[i]);
+__device__ __forceinline__ uint4 norm16(const uint4& x, const uint4& gamma, const uint4& beta, float2 st) {
+  const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, gw[4] = {gamma.x, gamma.y, gamma.z, gamma.w};
+  const uint32_t bw[4] = {beta.x, beta.y, beta.z, beta.w};
+  uint32_t r[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (DT == SKV_F32) {
+      r[i] = __float_as_uint(
+          fmaf((__uint_as_float(xw[i]) - st.x) * st.y, __uint_as_float(gw[i]), __uint_as_float(bw[i])));
+    } else {
+      r[i] = pack2<DT>(fmaf(fmaf(lo16<DT>(xw[i]), st.y, st.x), lo16<DT>(gw[i]), lo16<DT>(bw[i])),
+                       fmaf(fmaf(hi16<DT>(xw[i]), st.y, st.x), hi16<DT>(gw[i]), hi16<DT>(bw[i])));
+    }
   }
+  return make_uint4(r[0], r[1], r[2], r[3]);
+}
+
+// Four elements as loaded, and their fp32 values.
+template <int DT> struct Quad { uint2 v; };
+template <> struct Quad<SKV_F32> { f32x4 v; };
+template <int DT>
+__device__ __forceinline__ Quad<DT> load_raw(const char* p, int64_t elt) {
+  return *reinterpret_cast<const Quad<DT>*>(p + elt * (DT == SKV_F32 ? 4 : 2));
+}
+template <int DT>
+__device__ __forceinline__ f32x4 widen(const Quad<DT>& q) {
+  if constexpr (DT == SKV_F32) {
+    return q.v;
+  } else {
+    return f32x4{lo16<DT>(q.v.x), hi16<DT>(q.v.x), lo16<DT>(q.v.y), hi16<DT>(q.v.y)};
+  }
+}
+template <int DT>
+__device__ __forceinline__ f32x4 load_quad(const char* p, int64_t elt) {
+  return widen<DT>(load_raw<DT>(p, elt));
+}
+template <int DT>
+__device__ __forceinline__ void store_quad(char* p, int64_t elt, const f32x4& v) {
+  if constexpr (DT == SKV_F32) {
+    *reinterpret_cast<f32x4*>(p + elt * 4) = v;
+  } else {
+    *reinterpret_cast<uint2*>(p + elt * 2) = make_uint2(pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3]));
+  }
+}
+// The value as it reads back from the tensor type.
+template <int DT>
+__device__ __forceinline__ f32x4 round_quad(const f32x4& v) {
+  if constexpr (DT == SKV_F32) {
+    return v;
+  } else {
+    const uint32_t a = pack2<DT>(v[0], v[1]), b = pack2<DT>(v[2], v[3]);
+    return f32x4{lo16<DT>(a), hi16<DT>(a), lo16<DT>(b), hi16<DT>(b)};
+  }
+}
+
+// Sum of N values in each of LANES adjacent lanes, value i of lane l standing at index l + i * LANES of the row: over the
+// indices equal modulo 32 in order, then a tree over the 32 sums, so the bits do not depend on LANES.
+template <int LANES, int N>
+__device__ __forceinline__ float sum_mod32(const float* v) {
+  constexpr int kClasses = 32 / LANES;
+  static_assert(N % kClasses == 0, "whole rounds of 32 indices");
+  float s[kClasses];
+#pragma unroll
+  for (int c = 0; c < kClasses; ++c) s[c] = v[c];
+#pragma unroll
+  for (int i = kClasses; i < N; ++i) s[i % kClasses] += v[i];
+#pragma unroll
+  for (int h = kClasses / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int c = 0; c < h; ++c) s[c] += s[c + h];
+  float x = s[0];
+  if constexpr (LANES >= 32) x += xor_lane<16>(x);
+  if constexpr (LANES >= 16) x += xor_lane<8>(x);
+  if constexpr (LANES >= 8) x += xor_lane<4>(x);
+  x += xor_lane<2>(x);
+  return x + xor_lane<1>(x);
 }
 
 // A workgroup of WAVES waves owns 16 MI rows x 16 NI columns of y over split_chunks chunks of k.
 // Grid: (weight tile mod 8, row tile, weight tile / 8 * splits + split).
-template <int DT, int MI, int NI, int WAVES, int R>
+//
+// NORM: x is the LayerNorm of the given rows. The projection that stored them left the sum and the squared deviations
+// of every 16 elements, so a workgroup has its rows' mean and variance from k / 16 pairs a row (one load ahead of the
+// x loads) and normalises in registers on the way to LDS; a launch of its own costs 2.0 (k = 256) to 2.7 us (1280).
+template <int DT, int MI, int NI, int WAVES, int R, bool NORM>
 __global__ __launch_bounds__(64 * WAVES) void proj_kernel(
     const char* __restrict__ x, const char* __restrict__ w, uint32_t ldx, uint32_t ldw, uint32_t x_bytes,
-    uint32_t w_bytes, uint32_t m, uint32_t n, uint32_t kbytes, uint32_t split_chunks, uint32_t splits, ProjEpilogue p) {
+    uint32_t w_bytes, uint32_t m, uint32_t n, uint32_t kbytes, uint32_t split_chunks, uint32_t splits, ProjNorm q,
+    ProjEpilogue p) {
   constexpr int kRows = 16 * (MI + NI);
   constexpr int kStage = WAVES * kRows * kStageRow;
   constexpr int kTiles = MI * NI;
@@ -124,21 +211,66 @@ __global__ __launch_bounds__(64 * WAVES) void proj_kernel(
 #pragma unroll
     for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  // NORM: 16 MI / WAVES rows of statistics per wave, kNormLanes lanes each.
+  constexpr int kElt = DT == SKV_F32 ? 4 : 2;
+  constexpr int kNormRows = 16 * MI / WAVES, kNormLanes = 64 / kNormRows;
+  constexpr int kNormLoads = (WAVES * R * (kChunkBytes / (16 * kElt)) + 31) / 32 * (32 / kNormLanes);
+  __shared__ float2 s_norm[NORM ? 16 * MI : 1];
+  [[maybe_unused]] const uint32_t groups = kbytes / (16 * kElt);
+  [[maybe_unused]] const uint32_t srow = wave * kNormRows + lane / kNormLanes, sl = lane % kNormLanes;
+  float2 st[NORM ? kNormLoads : 1];
+  __amdgpu_buffer_rsrc_t gres, bres;
+  if constexpr (NORM) {
+    const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float2*>(q.stats), (short)0, (int)(m * groups * 8u), kBufWord3);
+    gres = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q.gamma), (short)0, (int)kbytes, kBufWord3);
+    bres = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q.beta), (short)0, (int)kbytes, kBufWord3);
+    const uint32_t row = m0 + srow;
+    const uint32_t base = row < m ? row * groups * 8u : kBufOutOfRange;
+#pragma unroll
+    for (int i = 0; i < kNormLoads; ++i) {
+      const uint32_t c = sl + i * kNormLanes;
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(sres, (base + c * 8u) | (c < groups ? 0u : kBufOutOfRange),
+                                                          0, 0);
+      st[i] = make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
+    }
+  }
+  // The epilogue's operands (thread's outputs: 4 columns of one row per trip), loaded ahead of the rows.
+  constexpr int kOut = (kTiles + WAVES - 1) / WAVES;
+  Quad<DT> bias[kOut] = {}, res[kOut] = {};
+#pragma unroll
+  for (int o = 0; o < kOut; ++o) {
+    const int tile = o * WAVES + wave;
+    const uint32_t mrow = m0 + 16 * (tile / NI) + r, ncol = n0 + 16 * (tile % NI) + 4 * g;
+    if (tile < kTiles && ncol < n) {
+      if (p.bias) bias[o] = load_raw<DT>(static_cast<const char*>(p.bias), ncol);
+      if (p.res && mrow < m) res[o] = load_raw<DT>(p.res, (int64_t)mrow * p.ldr + ncol);
+    }
+  }
   uint4 wr[R][2 * NI], xr[R][2 * MI];
+  uint4 gr[NORM ? R : 1], br[NORM ? R : 1];
+  float2 rowst[2 * MI];
   auto issue = [&](uint32_t k0, int s) __attribute__((always_inline)) {
     const uint32_t past = k0 + nat_col < k_end ? 0u : kBufOutOfRange;
 #pragma unroll
     for (int j = 0; j < 2 * NI; ++j) wr[s][j] = load_cached(wres, (woff[j] + k0) | past);
 #pragma unroll
     for (int j = 0; j < 2 * MI; ++j) xr[s][j] = load_cached(xres, (xoff[j] + k0) | past);
+    if constexpr (NORM) {
+      gr[s] = load_cached(gres, (k0 + nat_col) | past);
+      br[s] = load_cached(bres, (k0 + nat_col) | past);
+    }
   };
   auto compute = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 2 * NI; ++j)
       *reinterpret_cast<uint4*>(stage + (8 * j + nat_row) * kStageRow + nat_col) = wr[s][j];
 #pragma unroll
-    for (int j = 0; j < 2 * MI; ++j)
-      *reinterpret_cast<uint4*>(stage + (16 * NI + 8 * j + nat_row) * kStageRow + nat_col) = xr[s][j];
+    for (int j = 0; j < 2 * MI; ++j) {
+      uint4 v = xr[s][j];
+      if constexpr (NORM) v = norm16<DT>(v, gr[s], br[s], rowst[j]);
+      *reinterpret_cast<uint4*>(stage + (16 * NI + 8 * j + nat_row) * kStageRow + nat_col) = v;
+    }
     __builtin_amdgcn_wave_barrier();
     uint4 a[NI][2];
 #pragma unroll
@@ -167,6 +299,22 @@ __global__ __launch_bounds__(64 * WAVES) void proj_kernel(
 #pragma unroll
   for (int s = 0; s < R - 1; ++s) issue(k0 + s * kRound, s);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NORM) {
+    float v[kNormLoads];
+#pragma unroll
+    for (int i = 0; i < kNormLoads; ++i) v[i] = st[i].x;  // pairs past the row read zeros
+    const float mean = sum_mod32<kNormLanes, kNormLoads>(v) * q.inv_k;
+#pragma unroll
+    for (int i = 0; i < kNormLoads; ++i) {
+      const float d = fmaf(-16.f, mean, st[i].x);  // 16 (group mean - row mean)
+      v[i] = sl + i * kNormLanes < groups ? fmaf(d * 0.0625f, d, st[i].y) : 0.f;
+    }
+    const float rstd = rsqrtf(sum_mod32<kNormLanes, kNormLoads>(v) * q.inv_k + q.eps);
+    if (sl == 0) s_norm[srow] = make_float2(DT == SKV_F32 ? mean : -mean * rstd, rstd);
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < 2 * MI; ++j) rowst[j] = s_norm[8 * j + nat_row];
+  }
   if (last) compute(R - 1);
 #pragma unroll
   for (int s = 0; s < R - 1; ++s) compute(s);
@@ -178,32 +326,37 @@ __global__ __launch_bounds__(64 * WAVES) void proj_kernel(
 #pragma unroll
     for (int j = 0; j < NI; ++j) red[(wave * kTiles + i * NI + j) * 64 + lane] = acc[i][j];
   __syncthreads();
-  for (int t = threadIdx.x; t < kTiles * 64; t += 64 * WAVES) {
+#pragma unroll
+  for (int o = 0; o < kOut; ++o) {
+    const int tile = o * WAVES + wave, t = tile * 64 + lane;
+    if (tile >= kTiles) break;
     f32x4 v = red[t];
 #pragma unroll
     for (int wv = 1; wv < WAVES; ++wv) v += red[wv * kTiles * 64 + t];
-    const int tile = t >> 6, tl = t & 63;
-    const uint32_t mrow = m0 + 16 * (tile / NI) + (tl & 15);
-    const uint32_t ncol = n0 + 16 * (tile % NI) + 4 * (tl >> 4);
-    if (mrow >= m || ncol >= n) continue;
+    const uint32_t mrow = m0 + 16 * (tile / NI) + r;
+    const uint32_t ncol = n0 + 16 * (tile % NI) + 4 * g;
+    const bool in = mrow < m && ncol < n;
     if (p.part) {
-      *reinterpret_cast<f32x4*>(p.part + ((int64_t)split * m + mrow) * n + ncol) = v;
+      if (in) *reinterpret_cast<f32x4*>(p.part + ((int64_t)split * m + mrow) * n + ncol) = v;
       continue;
     }
-    if (p.bias) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += load_elt<DT>(p.bias, ncol + e);
-    }
+    v += widen<DT>(bias[o]);
     if (p.act) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = 0.5f * v[e] * (1.f + erff(v[e] * 0.70710678118654752f));
     }
-    const int64_t o = (int64_t)mrow * p.ldy + ncol;
-    if constexpr (DT == SKV_F32) {
-      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.y) + o) = v;
-    } else {
-      *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.y) + o) =
-          make_uint2(pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3]));
+    v += widen<DT>(res[o]);
+    v = round_quad<DT>(v);
+    if (in) store_quad<DT>(p.y, (int64_t)mrow * p.ldy + ncol, v);
+    if (p.stats) {  // n is a multiple of 16; the four lanes of a row's 16 elements, every lane active
+      float s16 = (v[0] + v[1]) + (v[2] + v[3]);
+      s16 += xor_lane<16>(s16);
+      s16 += xor_lane<32>(s16);
+      const f32x4 d = v - s16 * 0.0625f;
+      float q16 = fmaf(d[0], d[0], d[1] * d[1]) + fmaf(d[2], d[2], d[3] * d[3]);
+      q16 += xor_lane<16>(q16);
+      q16 += xor_lane<32>(q16);
+      if (in && g == 0) p.stats[(int64_t)mrow * (n / 16) + ncol / 16] = make_float2(s16, q16);
     }
   }
 }
@@ -233,34 +386,6 @@ struct AddNormParams {
   int32_t quads, splits;
   float eps, inv_n;
 };
-
-template <int DT>
-__device__ __forceinline__ f32x4 load_quad(const char* p, int64_t elt) {
-  if constexpr (DT == SKV_F32) {
-    return *reinterpret_cast<const f32x4*>(p + elt * 4);
-  } else {
-    const uint2 v = *reinterpret_cast<const uint2*>(p + elt * 2);
-    return f32x4{lo16<DT>(v.x), hi16<DT>(v.x), lo16<DT>(v.y), hi16<DT>(v.y)};
-  }
-}
-template <int DT>
-__device__ __forceinline__ void store_quad(char* p, int64_t elt, const f32x4& v) {
-  if constexpr (DT == SKV_F32) {
-    *reinterpret_cast<f32x4*>(p + elt * 4) = v;
-  } else {
-    *reinterpret_cast<uint2*>(p + elt * 2) = make_uint2(pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3]));
-  }
-}
-// The value as it reads back from the tensor type.
-template <int DT>
-__device__ __forceinline__ f32x4 round_quad(const f32x4& v) {
-  if constexpr (DT == SKV_F32) {
-    return v;
-  } else {
-    const uint32_t a = pack2<DT>(v[0], v[1]), b = pack2<DT>(v[2], v[3]);
-    return f32x4{lo16<DT>(a), hi16<DT>(a), lo16<DT>(b), hi16<DT>(b)};
-  }
-}
 
 // Sum over the workgroup; every thread gets the same bits. `slot` holds one float per wave.
 __device__ __forceinline__ float block_sum(float v, float* slot, int waves) {
@@ -324,11 +449,16 @@ void launch_add_norm(const AddNormParams& p, int rows, int32_t dtype, hipStream_
 constexpr int kDecodeRows = 128;
 constexpr int kMaxRows = 512;
 constexpr int kMinChunks = 4;             // 512-byte rows: a chunk for each wave
-constexpr uint32_t kMaxSplitChunks = 32;  // chunks of one workgroup: 8 waves x 4
+constexpr uint32_t kMaxChunks = 32;       // 4 KiB rows: 8 waves x 4, and every tile's registers
+// Rows of up to 6 KiB stay in one workgroup too (8 waves x 6, tiles of at most 32 x 32), so that the residual goes into
+// the epilogue and the launch that sums partials (2.3-2.9 us) falls away: 768 x 3072 bf16, 64 rows, with the residual
+// 5.0 us; a 12-layer step of that shape 1099 -> 1089 us, a 384-wide fp32 layer 42.1 -> 41.4 (with norm16's fma).
+constexpr uint32_t kMaxSplitChunks = 48;
 
 struct ProjShape {
   uint32_t m, n, kbytes, chunks, splits, split_chunks;
   int mi, ni, waves, rounds;
+  bool one_each;  // at most one workgroup per compute unit
 };
 
 // Compute units of the current device (256 when the query fails).
@@ -343,7 +473,7 @@ int compute_units() {
   return n;
 }
 
-int proj_splits(int64_t chunks) { return (int)cdiv(chunks, kMaxSplitChunks); }
+int proj_splits(int64_t chunks) { return chunks <= kMaxSplitChunks ? 1 : (int)cdiv(chunks, kMaxChunks); }
 
 // The contraction's split over workgroups, waves and rounds depends on k and the dtype alone, so a row's
 // bits do not depend on the batch it is in.
@@ -361,41 +491,52 @@ void pick_shape(ProjShape& p, int32_t m, int32_t n, int32_t kbytes) {
   const int tiles[4][2] = {{1, 1}, {2, 1}, {2, 2}, {4, 2}};
   const int64_t cus = compute_units();
   p.mi = p.ni = 2;
+  p.one_each = false;
   for (const auto& t : tiles) {
     if (t[0] > 1 && 8 * t[0] >= m) continue;  // half the tile's rows would be empty
+    if (t[0] > 2 && p.split_chunks > kMaxChunks) continue;
     if (cdiv(m, 16 * t[0]) * cdiv(n, 16 * t[1]) * p.splits <= cus) {
       p.mi = t[0], p.ni = t[1];
+      p.one_each = true;
       break;
     }
   }
 }
 
-template <int DT, int MI, int NI>
+template <int DT, int MI, int NI, bool NORM>
 void launch_tile(const ProjShape& s, const char* x, const char* w, uint32_t ldx, uint32_t ldw, uint32_t xb,
-                 uint32_t wb, const ProjEpilogue& e, hipStream_t st) {
+                 uint32_t wb, const ProjNorm& q, const ProjEpilogue& e, hipStream_t st) {
   const dim3 grid(8, (uint32_t)cdiv(s.m, 16 * MI), (uint32_t)(cdiv(s.n, 8 * 16 * NI) * s.splits));
 #define SKV_PROJ(W, R)                                                                                            \
-  hipLaunchKernelGGL((proj_kernel<DT, MI, NI, W, R>), grid, dim3(64 * W), 0, st, x, w, ldx, ldw, xb, wb, s.m, s.n, \
-                     s.kbytes, s.split_chunks, s.splits, e)
+  hipLaunchKernelGGL((proj_kernel<DT, MI, NI, W, R, NORM>), grid, dim3(64 * W), 0, st, x, w, ldx, ldw, xb, wb, s.m, \
+                     s.n, s.kbytes, s.split_chunks, s.splits, q, e)
   switch (s.waves * 4 + s.rounds) {
     case 17: SKV_PROJ(4, 1); break;
     case 18: SKV_PROJ(4, 2); break;
     case 19: SKV_PROJ(4, 3); break;
     case 34: SKV_PROJ(8, 2); break;
     case 35: SKV_PROJ(8, 3); break;
-    default: SKV_PROJ(8, 4); break;
+    case 36: SKV_PROJ(8, 4); break;
+    default:
+      if constexpr (MI <= 2 && !NORM) {
+        if (s.rounds == 5)
+          SKV_PROJ(8, 5);
+        else
+          SKV_PROJ(8, 6);
+      }
   }
 #undef SKV_PROJ
 }
 
-template <int DT>
+template <int DT, bool NORM>
 void launch_proj(const ProjShape& s, const char* x, const char* w, uint32_t ldx, uint32_t ldw, uint32_t xb,
-                 uint32_t wb, const ProjEpilogue& e, hipStream_t st) {
+                 uint32_t wb, const ProjNorm& q, const ProjEpilogue& e, hipStream_t st) {
   switch (s.mi * 4 + s.ni) {
-    case 5: launch_tile<DT, 1, 1>(s, x, w, ldx, ldw, xb, wb, e, st); break;
-    case 9: launch_tile<DT, 2, 1>(s, x, w, ldx, ldw, xb, wb, e, st); break;
-    case 10: launch_tile<DT, 2, 2>(s, x, w, ldx, ldw, xb, wb, e, st); break;
-    default: launch_tile<DT, 4, 2>(s, x, w, ldx, ldw, xb, wb, e, st); break;
+    case 5: launch_tile<DT, 1, 1, NORM>(s, x, w, ldx, ldw, xb, wb, q, e, st); break;
+    case 9: launch_tile<DT, 2, 1, NORM>(s, x, w, ldx, ldw, xb, wb, q, e, st); break;
+    case 10: launch_tile<DT, 2, 2, NORM>(s, x, w, ldx, ldw, xb, wb, q, e, st); break;
+    default:
+      if constexpr (!NORM) launch_tile<DT, 4, 2, NORM>(s, x, w, ldx, ldw, xb, wb, q, e, st);
   }
 }
 
@@ -410,7 +551,7 @@ int prepare_proj(const char* who, ProjShape& s, const void* x, int64_t ldx, cons
   const int64_t kb = (int64_t)k * eb;
   const int64_t xr = m > 0 ? (int64_t)(m - 1) * ldx * eb + kb : kb, wr = (int64_t)(n - 1) * ldw * eb + kb;
   const int64_t chunks = cdiv(kb, kChunkBytes);
-  const bool batch_ok = m <= kDecodeRows || (m <= kMaxRows && proj_splits(chunks) == 1 &&
+  const bool batch_ok = m <= kDecodeRows || (m <= kMaxRows && chunks <= kMaxChunks &&
                                              (int64_t)m * n <= (int64_t)1 << (eb == 4 ? 18 : 20));
   if (!batch_ok || n % 4 || kb % 16 || kb < kMinChunks * kChunkBytes || ldx * eb % 16 || ldw * eb % 16 ||
       xr > 0x7fffffff || wr > 0x7fffffff || kb > (int64_t)kMaxSplitChunks * kChunkBytes * 64)
@@ -422,15 +563,21 @@ int prepare_proj(const char* who, ProjShape& s, const void* x, int64_t ldx, cons
 }
 
 int run_proj(const char* who, const ProjShape& s, const void* x, int64_t ldx, const void* w, int64_t ldw, int32_t dtype,
-             uint32_t xb, uint32_t wb, const ProjEpilogue& e, hipStream_t st) {
+             uint32_t xb, uint32_t wb, const ProjNorm& q, const ProjEpilogue& e, hipStream_t st) {
   const uint32_t eb = (uint32_t)elt_bytes(dtype);
   const uint32_t lx = s.m > 1 ? (uint32_t)ldx * eb : s.kbytes, lw = s.n > 1 ? (uint32_t)ldw * eb : s.kbytes;
   const char *xp = (const char*)x, *wp = (const char*)w;
+#define SKV_PROJ_DT(DT)                                                \
+  if (q.gamma)                                                         \
+    launch_proj<DT, true>(s, xp, wp, lx, lw, xb, wb, q, e, st);        \
+  else                                                                 \
+    launch_proj<DT, false>(s, xp, wp, lx, lw, xb, wb, q, e, st);
   switch (dtype) {
-    case SKV_F32: launch_proj<SKV_F32>(s, xp, wp, lx, lw, xb, wb, e, st); break;
-    case SKV_F16: launch_proj<SKV_F16>(s, xp, wp, lx, lw, xb, wb, e, st); break;
-    default: launch_proj<SKV_BF16>(s, xp, wp, lx, lw, xb, wb, e, st); break;
+    case SKV_F32: SKV_PROJ_DT(SKV_F32) break;
+    case SKV_F16: SKV_PROJ_DT(SKV_F16) break;
+    default: SKV_PROJ_DT(SKV_BF16) break;
   }
+#undef SKV_PROJ_DT
   return check_launch(who);
 }
 
@@ -443,21 +590,46 @@ int32_t skv_decode_linear_splits(int32_t k, int32_t dtype) {
 
 int skv_decode_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, int32_t act, void* y,
                       int64_t ldy, int32_t m, int32_t n, int32_t k, int32_t dtype, void* stream) {
+  return skv_decode_linear_fused(x, ldx, nullptr, nullptr, nullptr, 0.f, w, ldw, bias, act, nullptr, 0, y, ldy, nullptr,
+                                 m, n, k, dtype, stream);
+}
+
+int skv_decode_linear_fused(const void* x, int64_t ldx, const float* x_stats, const void* gamma, const void* beta,
+                            float eps, const void* w, int64_t ldw, const void* bias, int32_t act, const void* res,
+                            int64_t ldr, void* y, int64_t ldy, float* y_stats, int32_t m, int32_t n, int32_t k,
+                            int32_t dtype, void* stream) {
+  const char* who = "skv_decode_linear";
   ProjShape s;
   uint32_t xb = 0, wb = 0;
-  const int rc = prepare_proj("skv_decode_linear", s, x, ldx, w, ldw, m, n, k, dtype, xb, wb);
+  const int rc = prepare_proj(who, s, x, ldx, w, ldw, m, n, k, dtype, xb, wb);
   if (rc != SKV_OK) return rc;
-  if (ldy < n || (act != 0 && act != SKV_ACT_GELU))
-    return fail(SKV_EINVAL, "skv_decode_linear: bad ldy=%lld (n=%d) or act=%d", (long long)ldy, n, act);
-  if (s.splits > 1 || ldy % 4)
-    return fail(SKV_EUNSUPPORTED, "skv_decode_linear: k=%d (dtype %d) is split over %u workgroups; ldy=%lld", k, dtype,
-                s.splits, (long long)ldy);
+  if (ldy < n || (res && ldr < n) || (act != 0 && act != SKV_ACT_GELU))
+    return fail(SKV_EINVAL, "%s: bad ldy=%lld, ldr=%lld (n=%d) or act=%d", who, (long long)ldy, (long long)ldr, n, act);
+  if (s.splits > 1 || ldy % 4 || (res && ldr % 4))
+    return fail(SKV_EUNSUPPORTED, "%s: k=%d (dtype %d) is split over %u workgroups; ldy=%lld ldr=%lld", who, k, dtype,
+                s.splits, (long long)ldy, (long long)ldr);
+  const bool norm = x_stats || gamma || beta;
+  if (norm && !(eps >= 0.f)) return fail(SKV_EINVAL, "%s: eps must be >= 0", who);
+  // Every workgroup normalises its rows again, so that pays where a unit has one workgroup of at most 32 rows (us, a
+  // LayerNorm launch and the plain projection / normalising; bf16): k = 1280, 64 rows, n = 3840 2.9 + 5.6 / 7.5, 1280
+  // 2.9 + 4.1 / 5.8; 128 rows, n = 1280 3.0 + 5.0 / 6.6; k = 768, 64 rows, n = 2304 2.6 + 4.2 / 5.6; k = 256 2.2 + 2.3 /
+  // 2.8. With 64-row tiles or more workgroups than units it does not: 64 rows, n = 5120 2.9 + 7.8 / 11.0, 128 rows
+  // 3.0 + 11.0 / 18.6.
+  const bool norm_ok = k % 16 == 0 && m <= kDecodeRows && s.one_each && s.mi <= 2 && s.chunks <= kMaxChunks;
+  if ((norm && !norm_ok) || (y_stats && n % 16))
+    return fail(SKV_EUNSUPPORTED, "%s: m=%d n=%d k=%d with row statistics", who, m, n, k);
   if (m == 0) return SKV_OK;
-  if (!x || !w || !y) return fail(SKV_EINVAL, "skv_decode_linear: null pointer argument");
-  if (!aligned16(x) || !aligned16(w) || ((uintptr_t)y & (4 * elt_bytes(dtype) - 1)))
-    return fail(SKV_EUNSUPPORTED, "skv_decode_linear: x and w rows must be 16-byte aligned");
-  ProjEpilogue e{bias, (char*)y, nullptr, ldy, act};
-  return run_proj("skv_decode_linear", s, x, ldx, w, ldw, dtype, xb, wb, e, (hipStream_t)stream);
+  if (!x || !w || !y || (norm && (!x_stats || !gamma || !beta)))
+    return fail(SKV_EINVAL, "%s: null pointer argument", who);
+  const uintptr_t quad = 4 * (uintptr_t)elt_bytes(dtype) - 1;
+  if (!aligned16(x) || !aligned16(w) || ((uintptr_t)y & quad) || ((uintptr_t)res & quad) || ((uintptr_t)bias & quad) ||
+      !aligned16(gamma) ||
+      !aligned16(beta) || ((uintptr_t)x_stats & 7) || ((uintptr_t)y_stats & 7))
+    return fail(SKV_EUNSUPPORTED, "%s: x, w, gamma and beta must be 16-byte aligned, y, res and bias to four elements",
+                who);
+  const ProjNorm q{gamma, beta, (const float2*)x_stats, eps, 1.f / (float)k};
+  const ProjEpilogue e{bias, (char*)y, nullptr, ldy, act, (const char*)res, ldr, (float2*)y_stats};
+  return run_proj(who, s, x, ldx, w, ldw, dtype, xb, wb, q, e, (hipStream_t)stream);
 }
 
 int skv_decode_linear_partials(const void* x, int64_t ldx, const void* w, int64_t ldw, float* part, int64_t part_floats,
@@ -473,8 +645,8 @@ int skv_decode_linear_partials(const void* x, int64_t ldx, const void* w, int64_
   if (part_floats < (int64_t)s.splits * m * n)
     return fail(SKV_EWORKSPACE, "skv_decode_linear_partials: part needs %lld floats, got %lld",
                 (long long)s.splits * m * n, (long long)part_floats);
-  ProjEpilogue e{nullptr, nullptr, part, 0, 0};
-  return run_proj("skv_decode_linear_partials", s, x, ldx, w, ldw, dtype, xb, wb, e, (hipStream_t)stream);
+  const ProjEpilogue e{nullptr, nullptr, part, 0, 0, nullptr, 0, nullptr};
+  return run_proj("skv_decode_linear_partials", s, x, ldx, w, ldw, dtype, xb, wb, ProjNorm{}, e, (hipStream_t)stream);
 }
 
 int skv_add_layernorm(const void* x, int64_t ldx, const void* y, int64_t ldy, const void* gamma, const void* beta,

@@ -246,31 +246,47 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] 
     return y
 
 
+def _plain(mod: nn.Module) -> bool:
+    return type(mod) is nn.Linear and not _hooked(mod)
+
+
 def proj(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """mod(x). A plain nn.Linear without hooks on a GPU tensor runs as one native projection (_linear); any other
     module, or one with hooks, is called as usual."""
-    if x.is_cuda and type(mod) is nn.Linear and not _hooked(mod):
+    if x.is_cuda and _plain(mod):
         return _linear(x, mod.weight, mod.bias)
     return mod(x)
+
+
+def _mlp_parts(seq: nn.Module, x: torch.Tensor):
+    """(fc1, act, fc2) of the layers' Linear-GELU-Linear MLP on a GPU tensor; None for another or a hooked module."""
+    if x.is_cuda and type(seq) is nn.Sequential and not _hooked(seq):
+        parts = tuple(seq._modules.values())
+        if len(parts) == 3 and type(parts[1]) is nn.GELU and not _hooked(parts[1]):
+            return parts
+    return None
 
 
 def _mlp(seq: nn.Module, x: torch.Tensor) -> Union[torch.Tensor, native.Partials]:
     """seq(x) for the layers' Linear-GELU-Linear MLP, its projections native (other modules and hooked ones are
     called as usual); the result as Partials when its last projection's contraction is split."""
-    if x.is_cuda and type(seq) is nn.Sequential and not _hooked(seq):
-        parts = tuple(seq._modules.values())
-        if len(parts) == 3 and type(parts[1]) is nn.GELU and not _hooked(parts[1]):
-            fc1, act, fc2 = parts
-            if act.approximate == "none" and type(fc1) is nn.Linear and not _hooked(fc1):
-                h = _linear(x, fc1.weight, fc1.bias, gelu=True)
-            else:
-                h = F.gelu(proj(fc1, x), approximate=act.approximate)
-            if type(fc2) is nn.Linear and not _hooked(fc2):
-                y = native.decode_partials(h, fc2.weight, fc2.bias)
-                if y is not None:
-                    return y
-            return proj(fc2, h)
-    return seq(x)
+    parts = _mlp_parts(seq, x)
+    if parts is None:
+        return seq(x)
+    fc1, act, fc2 = parts
+    if act.approximate == "none" and _plain(fc1):
+        h = _linear(x, fc1.weight, fc1.bias, gelu=True)
+    else:
+        h = F.gelu(proj(fc1, x), approximate=act.approximate)
+    return _mlp_out(fc2, h)
+
+
+def _mlp_out(fc2: nn.Module, h: torch.Tensor) -> Union[torch.Tensor, native.Partials]:
+    if _plain(fc2):
+        y = native.decode_partials(h, fc2.weight, fc2.bias)
+        if y is not None:
+            return y
+    return proj(fc2, h)
 
 
 def _tensor(y: Union[torch.Tensor, native.Partials]) -> torch.Tensor:
@@ -297,6 +313,40 @@ def add_norm(x: torch.Tensor, y: Union[torch.Tensor, native.Partials, None],
                 return got
     s = x if y is None else x + _tensor(y)
     return s, norm(s)
+
+
+class Residual:
+    """The residual stream between two blocks of a decoder layer: x + y, with y (a projection's result) not yet added
+    when there is one; stats: the statistics of x's rows (native.decode_linear_residual) when y has been added by the
+    projection itself, whose next projection then normalises x on its own (native.decode_linear_normed)."""
+
+    __slots__ = ("x", "y", "stats")
+
+    def __init__(self, x: torch.Tensor, y: Union[torch.Tensor, native.Partials, None] = None,
+                 stats: Optional[torch.Tensor] = None):
+        self.x, self.y, self.stats = x, y, stats
+
+    def add(self, mod: nn.Module, a: torch.Tensor) -> "Residual":
+        """The stream with mod(a) added; nothing of this stream may be pending."""
+        if a.is_cuda and _plain(mod):
+            got = native.decode_linear_residual(a, mod.weight, mod.bias, self.x)
+            if got is not None:
+                return Residual(got[0], None, got[1])
+        return Residual(self.x, proj(mod, a))
+
+    def normed_linear(self, norm: nn.Module, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                      gelu: bool = False) -> Optional[torch.Tensor]:
+        """act(norm(x) @ weight.T (+ bias)) as one launch, or None."""
+        if self.stats is None or type(norm) is not nn.LayerNorm or norm.weight is None or norm.bias is None or \
+                _hooked(norm):
+            return None
+        return native.decode_linear_normed(self.x, self.stats, norm.weight, norm.bias, norm.eps, weight, bias, gelu)
+
+    def normed(self, norm: nn.Module) -> torch.Tensor:
+        """norm(x + y), with y added into the stream."""
+        self.x, h = add_norm(self.x, self.y, norm)
+        self.y = None
+        return h
 
 
 @torch.no_grad()
@@ -364,9 +414,11 @@ class DecoderLayer(nn.Module):
 
     def _qkv_normed(self, h: torch.Tensor):
         """q, k, v [B, S, H, D] from the already normalised input h."""
-        b, s, _ = h.shape
+        return self._split_qkv(_linear(h, self.qkv_weight()) if h.is_cuda else F.linear(h, self.qkv_weight()))
+
+    def _split_qkv(self, qkv: torch.Tensor):
+        b, s, _ = qkv.shape
         hd = self.num_heads * self.head_dim
-        qkv = _linear(h, self.qkv_weight()) if h.is_cuda else F.linear(h, self.qkv_weight())
         shape = (b, s, self.num_heads, self.head_dim)
         return qkv[..., :hd].view(shape), qkv[..., hd:2 * hd].view(shape), qkv[..., 2 * hd:].view(shape)
 
@@ -385,30 +437,47 @@ class DecoderLayer(nn.Module):
         (pending: the previous layer's MLP output, not yet added). Returns (x, mlp
         output) with the MLP output left for the next layer (or the final norm) to
         add, so every residual add shares a launch with the LayerNorm that follows it."""
-        x, y = self._step_paged(x, layer, kv, cross, pending)
-        return x, _tensor(y)
+        r = self._step_paged(Residual(x, pending), layer, kv, cross)
+        return r.x, _tensor(r.y)
 
-    def _step_paged(self, x: torch.Tensor, layer: int, kv: PagedKV, cross: Optional[CrossKV],
-                    pending: Union[torch.Tensor, native.Partials, None]):
-        """forward_paged with the MLP output in and out as the projection left it (_mlp)."""
-        b, s, _ = x.shape
+    def _step_paged(self, r: Residual, layer: int, kv: PagedKV, cross: Optional[CrossKV], add: bool = False) -> Residual:
+        """forward_paged on the stream as the projections leave it; add: the MLP's output may be added already."""
+        b, s, _ = r.x.shape
         hd = self.num_heads * self.head_dim
-        x, h = add_norm(x, pending, self.norm1)
-        q, k, v = self._qkv_normed(h)
+        qkv = r.normed_linear(self.norm1, self.qkv_weight())
+        q, k, v = self._qkv_normed(r.normed(self.norm1)) if qkv is None else self._split_qkv(qkv)
         attn = native.paged_attention(q, kv.k_pools[layer], kv.v_pools[layer], kv.block_tables, kv.ctx_lens,
                                       kv.max_ctx, self.scale, causal=s > 1, table_rows=kv.table_rows,
                                       k_new=k, v_new=v, rows_longest_first=kv.rows_longest_first)
-        a = proj(self.self_attn_out, attn.view(b, s, hd))
-        used = cross is not None and cross.has(layer)
-        if used:
-            x, h = add_norm(x, a, self.norm2)
-            cq = proj(self.cross_attn_q, h).view(b, s, self.num_heads, self.head_dim)
-            c = native.dense_attention(cq, cross.k[layer], cross.v[layer], cross.lens,
-                                       cross.max_len, self.scale, slot_ids=cross.slot_ids)
-            x, h = add_norm(x, proj(self.cross_attn_out, c.view(b, s, hd)), self.norm3)
-        else:
-            x, h = add_norm(x, a, self.norm2)
-        return x, _mlp(self.mlp, h)
+        r = r.add(self.self_attn_out, attn.view(b, s, hd))
+        norm = self.norm2
+        if cross is not None and cross.has(layer):
+            cq = None
+            if _plain(self.cross_attn_q):
+                cq = r.normed_linear(norm, self.cross_attn_q.weight, self.cross_attn_q.bias)
+            if cq is None:
+                cq = proj(self.cross_attn_q, r.normed(norm))
+            c = native.dense_attention(cq.view(b, s, self.num_heads, self.head_dim), cross.k[layer], cross.v[layer],
+                                       cross.lens, cross.max_len, self.scale, slot_ids=cross.slot_ids)
+            r = r.add(self.cross_attn_out, c.view(b, s, hd))
+            norm = self.norm3
+        return self._mlp_paged(r, norm, add)
+
+    def _mlp_paged(self, r: Residual, norm: nn.Module, add: bool) -> Residual:
+        parts = _mlp_parts(self.mlp, r.x)
+        h = None
+        if parts is not None and parts[1].approximate == "none" and _plain(parts[0]):
+            h = r.normed_linear(norm, parts[0].weight, parts[0].bias, gelu=True)
+            if h is None:
+                h = _linear(r.normed(norm), parts[0].weight, parts[0].bias, gelu=True)
+        if h is None:
+            h = r.normed(norm)
+            return Residual(r.x, _mlp(self.mlp, h))
+        fc2 = parts[2]
+        if not add or not _plain(fc2):
+            return Residual(r.x, _mlp_out(fc2, h))
+        y = native.decode_partials(h, fc2.weight, fc2.bias)
+        return r.add(fc2, h) if y is None else Residual(r.x, y)
 
     # -- contiguous API of the reference (models.py:110-208) ---------------------
     def forward(self, x: torch.Tensor, past_key_values: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
@@ -463,14 +532,20 @@ class DecoderLayer(nn.Module):
         return self._finish(x, used), new_past, new_cross
 
 
-def _layer_step(layer: nn.Module, x: torch.Tensor, index: int, kv: PagedKV, cross: Optional[CrossKV],
-                pending: Union[torch.Tensor, native.Partials, None]):
-    """layer.forward_paged, its MLP output handed on as the projection left it; a layer whose forward_paged is
-    overridden is called through it, with tensors."""
+def _layer_step(layer: nn.Module, r: Residual, index: int, kv: PagedKV, cross: Optional[CrossKV]) -> Residual:
+    """layer.forward_paged on the stream, its MLP output added or handed on as the projection left it; a layer whose
+    forward_paged is overridden is called through it, with tensors."""
     if getattr(type(layer), "forward_paged", None) is DecoderLayer.forward_paged and \
             "forward_paged" not in layer.__dict__:
-        return layer._step_paged(x, index, kv, cross, pending)
-    return layer.forward_paged(x, index, kv, cross, None if pending is None else _tensor(pending))
+        return layer._step_paged(r, index, kv, cross, add=True)
+    return Residual(*layer.forward_paged(r.x, index, kv, cross, None if r.y is None else _tensor(r.y)))
+
+
+def _last_normed(r: Residual, last_only: bool, norm: nn.Module) -> torch.Tensor:
+    """norm of the stream (of its last position only, if last_only)."""
+    if last_only and r.x.shape[1] > 1:
+        r = Residual(r.x[:, -1:], None if r.y is None else _tensor(r.y)[:, -1:])
+    return r.normed(norm)
 
 
 # ---------------------------------------------------------------------------
@@ -553,14 +628,10 @@ class WhisperClassSpeechEncoderDecoderModel(nn.Module):
         """Run the decoder on input_ids [B, Q] whose K/V go into the paged pool at
         positions ctx_lens-Q .. ctx_lens-1; returns logits [B, V] of the last
         position (or [B, Q, V])."""
-        x = self._embed(input_ids)
-        pending = None
+        r = Residual(self._embed(input_ids))
         for l, layer in enumerate(self.decoder_layers):
-            x, pending = _layer_step(layer, x, l, kv, cross, pending)
-        if last_only and x.shape[1] > 1:
-            x = x[:, -1:]
-            pending = None if pending is None else _tensor(pending)[:, -1:]
-        _, h = add_norm(x, pending, self.decoder_norm)
+            r = _layer_step(layer, r, l, kv, cross)
+        h = _last_normed(r, last_only, self.decoder_norm)
         return proj(self.lm_head, h[:, 0] if last_only else h)
 
     # -- decode step, reference signature (models.py:369-423) ----------------------------
@@ -837,13 +908,8 @@ class StreamingMultiCodebookTTSModel(nn.Module):
         """Run the model on input_codebooks [B, Q, K] whose K/V go into the paged pool at
         positions ctx_lens-Q .. ctx_lens-1 (causal among the Q frames); returns the logits
         of the last frame [B, K, V] (or of every frame, [B, Q, K, V])."""
-        x = self.embeddings(input_codebooks)
-        pending = None
+        r = Residual(self.embeddings(input_codebooks))
         for l, layer in enumerate(self.layers):
-            x, pending = _layer_step(layer, x, l, kv, None, pending)
-        if last_only and x.shape[1] > 1:
-            x = x[:, -1:]
-            pending = None if pending is None else _tensor(pending)[:, -1:]
-        _, h = add_norm(x, pending, self.norm)
-        logits = self.heads(h)
+            r = _layer_step(layer, r, l, kv, None)
+        logits = self.heads(_last_normed(r, last_only, self.norm))
         return logits[:, 0] if last_only else logits

@@ -64,6 +64,8 @@ SIGNATURES = {
     "skv_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_p]),
     "skv_decode_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_i64, _c_i32, _c_i32, _c_i32,
                                    _c_i32, _c_p]),
+    "skv_decode_linear_fused": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_f, _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_i64,
+                                         _c_p, _c_i64, _c_p, _c_i32, _c_i32, _c_i32, _c_i32, _c_p]),
     "skv_decode_linear_splits": (_c_i32, [_c_i32, _c_i32]),
     "skv_decode_linear_partials": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
                                             _c_p]),
@@ -659,6 +661,53 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
     if rc == SKV_EUNSUPPORTED:
         return None
     _check(rc, "skv_decode_linear")
+    return y
+
+
+def decode_linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
+                           res: torch.Tensor) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """(s, stats): s = res + x @ weight.T (+ bias) of a decode batch, summed in fp32 and rounded once, and the statistics
+    of its rows that decode_linear_normed takes. None for a call that is not a decode projection."""
+    ops = _proj_operands(x, weight, bias)
+    if ops is None or res.dtype != x.dtype or res.shape != x.shape[:-1] + weight.shape[:1] or not res.is_cuda:
+        return None
+    x2, m, n, k, code = ops
+    r2 = res.reshape(m, n)
+    if n % 16 or r2.stride(1) != 1:
+        return None
+    y = torch.empty(res.shape, dtype=x.dtype, device=x.device)
+    stats = torch.empty((m, n // 16, 2), dtype=torch.float32, device=x.device)
+    rc = lib().skv_decode_linear_fused(x2.data_ptr(), x2.stride(0) if m > 1 else k, None, None, None, 0.0,
+                                       weight.data_ptr(), weight.stride(0) if n > 1 else k, _ptr(bias), SKV_ACT_NONE,
+                                       r2.data_ptr(), r2.stride(0) if m > 1 else n, y.data_ptr(), n, stats.data_ptr(),
+                                       m, n, k, code, _stream(x.device))
+    if rc == SKV_EUNSUPPORTED:
+        return None
+    _check(rc, "skv_decode_linear_fused")
+    return y, stats
+
+
+def decode_linear_normed(x: torch.Tensor, stats: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, eps: float,
+                         weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                         gelu: bool = False) -> Optional[torch.Tensor]:
+    """act(LayerNorm(x) @ weight.T (+ bias)) of a decode batch in one launch; stats are those of x's rows
+    (decode_linear_residual). None for a call that is not a decode projection."""
+    ops = _proj_operands(x, weight, bias)
+    if ops is None:
+        return None
+    x2, m, n, k, code = ops
+    for t in (gamma, beta):
+        if t.dtype != x.dtype or t.shape != (k,) or t.stride(0) != 1 or not t.is_cuda:
+            return None
+    y = torch.empty(x.shape[:-1] + (n,), dtype=x.dtype, device=x.device)
+    rc = lib().skv_decode_linear_fused(x2.data_ptr(), x2.stride(0) if m > 1 else k, stats.data_ptr(), gamma.data_ptr(),
+                                       beta.data_ptr(), float(eps), weight.data_ptr(),
+                                       weight.stride(0) if n > 1 else k, _ptr(bias),
+                                       SKV_ACT_GELU if gelu else SKV_ACT_NONE, None, 0, y.data_ptr(), n, None, m, n, k,
+                                       code, _stream(x.device))
+    if rc == SKV_EUNSUPPORTED:
+        return None
+    _check(rc, "skv_decode_linear_fused")
     return y
 
 

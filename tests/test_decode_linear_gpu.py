@@ -1,7 +1,7 @@
 """Decode-batch projections (skv_decode_linear, its partials, skv_reduce_add_layernorm) against float64.
 
 Sizes sit at the edges of the kernel's tiles (16 to 64 rows, 16 or 32 columns), of its 128-byte chunks and of its
-split (4 KiB rows). The bar is the output's rounding plus the fp32 accumulation bound k * 2^-24 * sum |x w|.
+split (6 KiB rows). The bar is the output's rounding plus the fp32 accumulation bound k * 2^-24 * sum |x w|.
 """
 import copy
 
@@ -34,15 +34,18 @@ def _check(y, ref, bound, what):
 
 
 # (m, n) around the row and column tiles and the one-workgroup-per-unit rule; k in elements of a 16-bit dtype:
-# 256 (one chunk per wave), 264 and 776 (partial last chunks), 1280 (8 waves, 3 rounds, a partial round), 2048 (4 rounds)
+# 256 (one chunk per wave), 264 and 776 (partial last chunks), 1280 (8 waves, 3 rounds, a partial round), 2048 (4 rounds),
+# 2056 and 3072 (5 and 6 rounds, tiles of at most 32 rows)
 MN = [(1, 4), (1, 1284), (9, 20), (16, 16), (17, 36), (33, 132), (64, 1280), (65, 3840), (128, 1056), (300, 260)]
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("k16", [256, 264, 776, 1280, 2048])
+@pytest.mark.parametrize("k16", [256, 264, 776, 1280, 2048, 2056, 3072])
 def test_decode_linear_against_float64(cuda, dt, k16):
     k = k16 if dt != torch.float32 else k16 // 2
     for m, n in MN:
+        if m > 128 and k16 > 2048:
+            continue  # a longer row takes a decode batch only
         x, w, b, ref, bound = _data(m, n, k, dt, m * 7 + n)
         _check(native.decode_linear(x, w, b), ref, bound, f"m={m} n={n} k={k}")
         y = native.decode_linear(x, w, b, gelu=True)
@@ -50,7 +53,7 @@ def test_decode_linear_against_float64(cuda, dt, k16):
         _check(y, F.gelu(ref), 1.13 * bound + 2.0 ** -20 * ref.abs(), f"gelu m={m} n={n} k={k}")
 
 
-@pytest.mark.parametrize("dt,k", [(torch.bfloat16, 2056), (torch.float16, 5120), (torch.float32, 1536)])
+@pytest.mark.parametrize("dt,k", [(torch.bfloat16, 3080), (torch.float16, 5120), (torch.float32, 1540)])
 def test_partials_and_reduce_add_layernorm(cuda, dt, k):
     for m, n in [(1, 256), (17, 384), (64, 1280), (128, 4096 if dt != torch.float32 else 2048)]:
         x, w, b, ref, bound = _data(m, n, k, dt, m + n)
@@ -113,3 +116,56 @@ def test_mlp_in_a_graph_replays(cuda):
             assert torch.equal(y, models.mlp(seq, x))
             want = seq64(x.double())
             assert float((y.double() - want).norm() / want.norm()) < 2 * EPS[dt]
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("d", [256, 384, 768, 1280])
+def test_residual_and_normed_projection(cuda, dt, d):
+    """A residual projection, then a projection of its LayerNorm, in one launch each."""
+    if dt == torch.float32 and d == 1280:
+        d = 1024  # the longest unsplit fp32 row
+    for m, n in [(1, 256), (4, 3 * d), (17, 512), (33, 1040), (64, 4 * d), (128, 4)]:
+        a, w, b, ref, bound = _data(m, d, d, dt, m + n)
+        g = torch.Generator(device="cuda").manual_seed(m)
+        res = (3 * torch.randn(m, d, generator=g, device="cuda") + 5).to(dt)  # a mean well off zero
+        s, stats = native.decode_linear_residual(a, w, b, res)
+        _check(s, ref + res.double(), bound + 2.0 ** -23 * (ref.abs() + res.double().abs()), f"residual m={m} d={d}")
+        grp = s.double().view(m, d // 16, 16)
+        assert torch.allclose(stats[..., 0].double(), grp.sum(-1), rtol=1e-5, atol=1e-4)
+        dev = (grp - grp.mean(-1, keepdim=True)).square().sum(-1)
+        assert torch.allclose(stats[..., 1].double(), dev, rtol=1e-5, atol=1e-4)
+        gm, bt = (torch.randn(d, generator=g, device="cuda").to(dt) for _ in range(2))
+        w2 = (torch.randn(n, d, generator=g, device="cuda") * d ** -0.5).to(dt)
+        b2 = torch.randn(n, generator=g, device="cuda").to(dt)
+        want = F.layer_norm(s.double(), (d,), gm.double(), bt.double(), 1e-5)
+        for gelu in (False, True):
+            y = native.decode_linear_normed(s, stats, gm, bt, 1e-5, w2, b2, gelu)
+            if y is None:  # a tile of 64 rows, or more workgroups than units
+                assert m * n > 16 * 256 * 16 * 4
+                break
+            ref2 = want @ w2.double().t() + b2.double()
+            # each normalised element rounded to dtype (and a few fp32 roundings), then the product's own bound
+            slack = (2 * EPS[dt] + (d + 8) * 2.0 ** -24) * (want.abs() + 1e-2) @ w2.double().abs().t() + 1e-6
+            _check(y, F.gelu(ref2) if gelu else ref2, 1.13 * slack + 2.0 ** -20 * ref2.abs(), f"normed m={m} n={n} d={d}")
+        full = native.decode_linear_normed(s, stats, gm, bt, 1e-5, w2, b2)
+        if full is None:
+            continue
+        assert torch.equal(native.decode_linear_normed(s[:1], stats[:1].contiguous(), gm, bt, 1e-5, w2, b2), full[:1])
+
+
+def test_fused_projection_refuses_what_it_does_not_take(cuda):
+    a, w, b, _, _ = _data(8, 512, 512, torch.bfloat16, 1)
+    res = torch.zeros(8, 512, device="cuda", dtype=torch.bfloat16)
+    assert native.decode_linear_residual(a, w[:500], None, res[:, :500]) is None  # columns not whole groups of 16
+    assert native.decode_linear_residual(a, w, None, res.float()) is None
+    assert native.decode_linear_residual(a, w, None, res[:4]) is None
+    big = torch.zeros(129, 512, device="cuda", dtype=torch.bfloat16)
+    s, st = native.decode_linear_residual(big, w, None, big)
+    assert native.decode_linear_normed(s, st, b, b, 1e-5, w) is None  # past the decode batch
+    assert native.decode_linear_normed(s[:8], st[:8], b[1:], b, 1e-5, w) is None
+    nan = a.clone()
+    nan[3, 7] = float("nan")  # reaches its own row only
+    s, st = native.decode_linear_residual(nan, w, b, res)
+    y = native.decode_linear_normed(s, st, b, b, 1e-5, w)
+    bad = torch.isnan(y).any(dim=1)
+    assert bool(bad[3]) and int(bad.sum()) == 1
