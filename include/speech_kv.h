@@ -397,6 +397,21 @@ SKV_API int skv_decode_linear_fused(const void* x, int64_t ldx, const float* x_s
                                     int32_t m, int32_t n, int32_t k, int32_t dtype, void* stream);
 
 /*
+ * skv_rows_linear — a projection of many rows (a prompt, a request's frames) on the matrix cores, 16-bit types:
+ *   y[r*ldy + j] = act(sum_i x[r*ldx + i] * w[j*ldw + i] (+ bias[j])) (+ res[r*ldr + j]); products, sums, activation and
+ *   residual in fp32, rounded once. bias, res: NULL for none (res may be y).
+ *   hd > 0: w is the q, k and v weights stacked (n = 3 hd); only columns below hd go to y, the k and v columns to k_out
+ *   and v_out [m / tokens, hd / 64, tokens, 64] (row r is token r % tokens of batch r / tokens); then res must be NULL.
+ * SKV_EUNSUPPORTED (nothing launched; the caller runs another GEMM): fp32, n or a row stride not a multiple of 8,
+ * k * 2 bytes not of whole 16-byte vectors, an unaligned pointer, x or w past 2 GiB, or a shape that the library's GEMM serves
+ * better.
+ * Replaces the nn.Linear (and GELU) calls of the encoder and the prefill, speech_serving/models.py:110-207.
+ */
+SKV_API int skv_rows_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, int32_t act,
+                            const void* res, int64_t ldr, void* y, int64_t ldy, void* k_out, void* v_out, int32_t hd,
+                            int32_t tokens, int32_t m, int32_t n, int32_t k, int32_t dtype, void* stream);
+
+/*
  * Workgroups that share the contraction of one output of a projection over k elements of dtype (1: none do,
  * skv_decode_linear writes the result itself). 0 for a bad argument.
  */

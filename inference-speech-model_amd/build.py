@@ -19,7 +19,7 @@ PKG_ROOT = os.path.dirname(os.path.abspath(__file__))
 REPO_ROOT = os.path.dirname(PKG_ROOT)
 CSRC = os.path.join(PKG_ROOT, "csrc")
 INCLUDE = os.path.join(REPO_ROOT, "include")
-SOURCES = [os.path.join(CSRC, f) for f in ("skv_kernels.hip", "skv_linear.hip", "skv_proj.hip")]
+SOURCES = [os.path.join(CSRC, f) for f in ("skv_kernels.hip", "skv_linear.hip", "skv_proj.hip", "skv_gemm.hip")]
 OUTPUT = os.path.join(PKG_ROOT, "speech_serving", "libspeechkv.so")
 ARCH = "gfx950"
 

@@ -236,9 +236,12 @@ def _hooked(mod: nn.Module) -> bool:
 
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
             gelu: bool = False) -> torch.Tensor:
-    """x @ weight.T (+ bias), then the erf GELU when gelu: a decode batch in one skv_decode_linear launch, other
-    shapes through skv_linear (a hipBLASLt plan cached per shape) and torch's GELU."""
+    """x @ weight.T (+ bias), then the erf GELU when gelu: a decode batch in one skv_decode_linear launch, more rows
+    with GELU in one skv_rows_linear launch, other shapes through skv_linear (a hipBLASLt plan cached per shape) and
+    torch's GELU."""
     y = native.decode_linear(x, weight, bias, gelu)
+    if y is None and gelu and x.numel() > native.DECODE_ROWS * x.shape[-1]:
+        y = native.rows_linear(x, weight, bias, gelu=True)
     if y is None:
         y = native.linear(x, weight, bias)
         if gelu:
@@ -315,6 +318,14 @@ def add_norm(x: torch.Tensor, y: Union[torch.Tensor, native.Partials, None],
     return s, norm(s)
 
 
+def _sum_norm(x: torch.Tensor, y: Optional[torch.Tensor], norm: nn.Module) -> Tuple[torch.Tensor, torch.Tensor]:
+    """add_norm, in torch's own ops where x takes part in autograd."""
+    if x.requires_grad or (y is not None and y.requires_grad):
+        s = x if y is None else x + y
+        return s, norm(s)
+    return add_norm(x, y, norm)
+
+
 class Residual:
     """The residual stream between two blocks of a decoder layer: x + y, with y (a projection's result) not yet added
     when there is one; stats: the statistics of x's rows (native.decode_linear_residual) when y has been added by the
@@ -328,7 +339,7 @@ class Residual:
 
     def add(self, mod: nn.Module, a: torch.Tensor) -> "Residual":
         """The stream with mod(a) added; nothing of this stream may be pending."""
-        if a.is_cuda and _plain(mod):
+        if a.is_cuda and _plain(mod) and a.numel() <= native.DECODE_ROWS * a.shape[-1]:
             got = native.decode_linear_residual(a, mod.weight, mod.bias, self.x)
             if got is not None:
                 return Residual(got[0], None, got[1])
@@ -487,15 +498,22 @@ class DecoderLayer(nn.Module):
                 encoder_attention_mask: Optional[torch.Tensor] = None):
         b, s, _ = x.shape
         hd = self.num_heads * self.head_dim
-        q, k, v = self._qkv(x)
-        k = k.transpose(1, 2)
-        v = v.transpose(1, 2)
-        if past_key_values is not None:
-            pk, pv = past_key_values
-            k = torch.cat([pk.to(q.dtype), k], dim=2)
-            v = torch.cat([pv.to(q.dtype), v], dim=2)
+        _, h = _sum_norm(x, None, self.norm1)
+        got = None
+        if past_key_values is None and b * s > native.DECODE_ROWS and self.head_dim == 64:
+            got = native.rows_qkv(h, self.qkv_weight(), self.num_heads)
+        if got is not None:
+            q, k, v = got
         else:
-            k, v = k.contiguous(), v.contiguous()
+            q, k, v = self._qkv_normed(h)
+            k = k.transpose(1, 2)
+            v = v.transpose(1, 2)
+            if past_key_values is not None:
+                pk, pv = past_key_values
+                k = torch.cat([pk.to(q.dtype), k], dim=2)
+                v = torch.cat([pv.to(q.dtype), v], dim=2)
+            else:
+                k, v = k.contiguous(), v.contiguous()
         new_past = (k, v)
         t = k.shape[2]
         if attention_mask is not None:
@@ -504,10 +522,9 @@ class DecoderLayer(nn.Module):
             kk, vv = k, v
             lens = torch.full((b,), t, dtype=torch.int32, device=x.device)
         attn = native.dense_attention(q, kk, vv, lens, t, self.scale, causal=self.is_decoder and s > 1)
-        x = x + proj(self.self_attn_out, attn.reshape(b, s, hd))
-
         new_cross = None
         used = encoder_hidden_states is not None or encoder_past_kv is not None
+        x, h = _sum_norm(x, proj(self.self_attn_out, attn.reshape(b, s, hd)), self.norm2)
         if used:
             if encoder_past_kv is not None:
                 ck, cv = encoder_past_kv
@@ -527,9 +544,10 @@ class DecoderLayer(nn.Module):
                 clens = torch.full((b,), te, dtype=torch.int32, device=x.device)
             if ck.shape[0] == 1 and b > 1:
                 ck, cv = ck.expand(b, -1, -1, -1), cv.expand(b, -1, -1, -1)
-            c = native.dense_attention(self._cross_q(x), ck, cv, clens, te, self.scale)
-            x = x + proj(self.cross_attn_out, c.reshape(b, s, hd))
-        return self._finish(x, used), new_past, new_cross
+            cq = proj(self.cross_attn_q, h).view(b, s, self.num_heads, self.head_dim)
+            c = native.dense_attention(cq, ck, cv, clens, te, self.scale)
+            x, h = _sum_norm(x, proj(self.cross_attn_out, c.reshape(b, s, hd)), self.norm3)
+        return x + mlp(self.mlp, h), new_past, new_cross
 
 
 def _layer_step(layer: nn.Module, r: Residual, index: int, kv: PagedKV, cross: Optional[CrossKV]) -> Residual:

@@ -13,6 +13,9 @@ Functions:
     linear(x, weight, bias)   (hipBLASLt with a plan cached per shape)
     decode_linear(x, weight, bias, gelu), decode_partials(x, weight, bias), reduce_add_layernorm(...)
                               (a decode batch's projections on the matrix cores)
+    decode_linear_residual(x, weight, bias, res), decode_linear_normed(x, stats, gamma, beta, eps, weight, ...)
+                              (with the residual add behind, or the LayerNorm ahead)
+    rows_linear(x, weight, bias, gelu, res), rows_qkv(x, weight, heads)   (many 16-bit rows)
 """
 from __future__ import annotations
 
@@ -66,6 +69,8 @@ SIGNATURES = {
                                    _c_i32, _c_p]),
     "skv_decode_linear_fused": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_f, _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_i64,
                                          _c_p, _c_i64, _c_p, _c_i32, _c_i32, _c_i32, _c_i32, _c_p]),
+    "skv_rows_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i32, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_i32,
+                                 _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_p]),
     "skv_decode_linear_splits": (_c_i32, [_c_i32, _c_i32]),
     "skv_decode_linear_partials": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
                                             _c_p]),
@@ -74,6 +79,7 @@ SIGNATURES = {
 }
 SKV_EUNSUPPORTED = -5  # skv_linear, skv_decode_linear: not a shape or layout the call takes
 SKV_ACT_NONE, SKV_ACT_GELU = 0, 1
+DECODE_ROWS = 128  # a decode batch (kDecodeRows of the library)
 MAX_DECODE_ROWS = 512  # most rows skv_decode_linear takes (kMaxRows of the library)
 MAX_CODEBOOKS = 16  # kMaxCodebooks of the library
 
@@ -627,13 +633,26 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     return y
 
 
-def _proj_operands(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]):
+def decode_batch(x: torch.Tensor, n: int) -> bool:
+    """Whether x [..., k] times n columns is a batch that skv_decode_linear takes (its own rule, asked before anything is
+    prepared): up to 128 rows, or up to 512 with few outputs."""
+    k = x.shape[-1]
+    size = x.numel()
+    if size <= DECODE_ROWS * k:
+        return True
+    wide = x.element_size() == 4
+    return size <= MAX_DECODE_ROWS * k and size * n <= (k << (18 if wide else 20)) and k <= (1024 if wide else 2048)
+
+
+def _proj_operands(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], max_rows: int):
     """(x as [m, k] rows, m, n, k, dtype code) of a decode projection, or None when the batch, the types or the
     layouts are not those skv_decode_linear takes (its own checks decide about sizes and alignment)."""
     k = x.shape[-1]
+    if x.numel() > max_rows * k:
+        return None
     code = _DTYPE_CODE.get(x.dtype)
     if code is None or not x.is_cuda or not weight.is_cuda or weight.dtype != x.dtype or weight.dim() != 2 or \
-            weight.shape[1] != k or weight.stride(1) != 1 or x.numel() > MAX_DECODE_ROWS * k or k == 0:
+            weight.shape[1] != k or weight.stride(1) != 1 or k == 0:
         return None
     n = weight.shape[0]
     if bias is not None and (bias.dtype != x.dtype or bias.dim() != 1 or bias.shape[0] != n or bias.stride(0) != 1
@@ -650,7 +669,7 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
     """act(x @ weight.T (+ bias)) of a decode batch (or a short prompt batch) in one launch on the matrix cores, summed
     in fp32 and rounded once; gelu applies the erf GELU to the fp32 result. None for a call skv_decode_linear does
     not take (the caller runs linear()). Reference: speech_serving/models.py:127-207."""
-    ops = _proj_operands(x, weight, bias)
+    ops = _proj_operands(x, weight, bias, MAX_DECODE_ROWS) if decode_batch(x, weight.shape[0]) else None
     if ops is None:
         return None
     x2, m, n, k, code = ops
@@ -668,7 +687,7 @@ def decode_linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: Optional
                            res: torch.Tensor) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
     """(s, stats): s = res + x @ weight.T (+ bias) of a decode batch, summed in fp32 and rounded once, and the statistics
     of its rows that decode_linear_normed takes. None for a call that is not a decode projection."""
-    ops = _proj_operands(x, weight, bias)
+    ops = _proj_operands(x, weight, bias, MAX_DECODE_ROWS)
     if ops is None or res.dtype != x.dtype or res.shape != x.shape[:-1] + weight.shape[:1] or not res.is_cuda:
         return None
     x2, m, n, k, code = ops
@@ -692,7 +711,7 @@ def decode_linear_normed(x: torch.Tensor, stats: torch.Tensor, gamma: torch.Tens
                          gelu: bool = False) -> Optional[torch.Tensor]:
     """act(LayerNorm(x) @ weight.T (+ bias)) of a decode batch in one launch; stats are those of x's rows
     (decode_linear_residual). None for a call that is not a decode projection."""
-    ops = _proj_operands(x, weight, bias)
+    ops = _proj_operands(x, weight, bias, MAX_DECODE_ROWS)
     if ops is None:
         return None
     x2, m, n, k, code = ops
@@ -709,6 +728,55 @@ def decode_linear_normed(x: torch.Tensor, stats: torch.Tensor, gamma: torch.Tens
         return None
     _check(rc, "skv_decode_linear_fused")
     return y
+
+
+def rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, gelu: bool = False,
+                res: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """act(x @ weight.T (+ bias)) (+ res) of many 16-bit rows in one launch on the matrix cores, summed in fp32 and rounded
+    once. None for a call skv_rows_linear does not take."""
+    ops = None if x.dtype == torch.float32 else _proj_operands(x, weight, bias, 1 << 30)
+    if ops is None:
+        return None
+    x2, m, n, k, code = ops
+    r2 = None
+    if res is not None:
+        if res.dtype != x.dtype or res.shape != x.shape[:-1] + (n,) or not res.is_cuda:
+            return None
+        r2 = res.reshape(m, n)
+        if r2.stride(1) != 1 or (m > 1 and r2.stride(0) < n):
+            return None
+    y = torch.empty(x.shape[:-1] + (n,), dtype=x.dtype, device=x.device)
+    rc = lib().skv_rows_linear(x2.data_ptr(), x2.stride(0) if m > 1 else k, weight.data_ptr(),
+                               weight.stride(0) if n > 1 else k, _ptr(bias), SKV_ACT_GELU if gelu else SKV_ACT_NONE,
+                               _ptr(r2), r2.stride(0) if r2 is not None and m > 1 else n, y.data_ptr(), n, None, None, 0,
+                               0, m, n, k, code, _stream(x.device))
+    if rc == SKV_EUNSUPPORTED:
+        return None
+    _check(rc, "skv_rows_linear")
+    return y
+
+
+def rows_qkv(x: torch.Tensor, weight: torch.Tensor,
+             heads: int) -> Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]]:
+    """q [B, S, H, 64], k and v [B, H, S, 64] (contiguous) of x [B, S, k] and the stacked q/k/v weight [3 * H * 64, k] in one
+    launch. None for a call skv_rows_linear does not take."""
+    hd = heads * 64
+    if x.dtype == torch.float32 or x.dim() != 3 or weight.dim() != 2 or weight.shape[0] != 3 * hd:
+        return None
+    ops = _proj_operands(x, weight, None, 1 << 30)
+    if ops is None or ops[1] == 0:
+        return None
+    x2, m, n, k, code = ops
+    b, s, _ = x.shape
+    q = torch.empty((b, s, heads, 64), dtype=x.dtype, device=x.device)
+    kk, vv = (torch.empty((b, heads, s, 64), dtype=x.dtype, device=x.device) for _ in range(2))
+    rc = lib().skv_rows_linear(x2.data_ptr(), x2.stride(0) if m > 1 else k, weight.data_ptr(),
+                               weight.stride(0) if n > 1 else k, None, SKV_ACT_NONE, None, 0, q.data_ptr(), hd,
+                               kk.data_ptr(), vv.data_ptr(), hd, s, m, n, k, code, _stream(x.device))
+    if rc == SKV_EUNSUPPORTED:
+        return None
+    _check(rc, "skv_rows_linear")
+    return q, kk, vv
 
 
 class Partials:
@@ -732,7 +800,7 @@ def _decode_splits(k: int, code: int) -> int:
 def decode_partials(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[Partials]:
     """x @ weight.T (+ bias) as Partials when the projection's contraction is split, else None (a call that
     decode_linear or linear takes)."""
-    ops = _proj_operands(x, weight, bias)
+    ops = _proj_operands(x, weight, bias, DECODE_ROWS)
     if ops is None:
         return None
     x2, m, n, k, code = ops
@@ -797,6 +865,31 @@ def _layernorm_rows(x: torch.Tensor, weight: torch.Tensor):
     return x2, h, epl
 
 
+def _add_layernorm_contiguous(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, bias: torch.Tensor,
+                              eps: float) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """add_layernorm of contiguous tensors, the layers' case, with as little host work as it takes; None for any other
+    case (the general path then decides)."""
+    dt = x.dtype
+    h = x.shape[-1]
+    code = _DTYPE_CODE.get(dt)
+    if code is None or not x.is_cuda or h == 0 or h % 8 or h > 2048 or weight.dtype != dt or bias.dtype != dt or \
+            weight.shape != (h,) or bias.shape != (h,) or not weight.is_contiguous() or not bias.is_contiguous() or \
+            x.data_ptr() % 16:
+        return None
+    s = x
+    yp = sp = None
+    if y is not None:
+        if y.dtype != dt or y.shape != x.shape or not y.is_contiguous() or not y.is_cuda or y.data_ptr() % 16:
+            return None
+        s = torch.empty_like(x)
+        yp, sp = y.data_ptr(), s.data_ptr()
+    norm = torch.empty_like(x)
+    rc = lib().skv_add_layernorm(x.data_ptr(), h, yp, h, weight.data_ptr(), bias.data_ptr(), float(eps), sp, h,
+                                 norm.data_ptr(), h, x.numel() // h, h, code, _stream(x.device))
+    _check(rc, "skv_add_layernorm")
+    return s, norm
+
+
 def add_layernorm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, bias: torch.Tensor,
                   eps: float, sum_out: Optional[torch.Tensor] = None,
                   fallback: bool = False) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
@@ -807,6 +900,10 @@ def add_layernorm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tens
     vector or above 512 of them, rows that are not 16-byte aligned, a weight or bias of another size)
     raises RuntimeError, or with fallback=True returns None (the caller then runs torch's ops).
     """
+    if sum_out is None and x.is_contiguous():
+        got = _add_layernorm_contiguous(x, y, weight, bias, eps)
+        if got is not None:
+            return got
     got = _layernorm_rows(x, weight)
     if got is not None and (not weight.is_contiguous() or weight.numel() != got[1] or bias.dtype != x.dtype or
                             not bias.is_contiguous() or bias.numel() != got[1]):
