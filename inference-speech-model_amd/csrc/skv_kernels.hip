@@ -1416,6 +1416,129 @@ __global__ __launch_bounds__(256) void merge_kernel(AttnParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// fp32 attention of many queries over contiguous K/V (an encoder layer, a prompt's cross-attention), head_dim 64, on
+// the matrix cores: one workgroup per (row, head, 16 queries), its waves take the keys in turns of 16 and merge at
+// the end. Everything stays in registers: the contraction index an element stands for only has to agree between the
+// operands, so lane (g, r) loads whole 64-byte pieces (key r, dims 16 g .. + 15; keys 4 g + e, dims 4 r .. + 3), and the
+// scores come out as the operand that the second product takes.
+// What bounds it: the 16 x 16 x 4 products (32 of 32 clocks each; 32 of them per 16 keys and wave). One workgroup per query read a head's
+// keys 16 times as often (1 x 600 queries, 12 heads, 600 keys: 110-140 us, now 21.8).
+// A key past the row's length reads zeros and its score is masked, so what the buffer holds there does not matter.
+// ---------------------------------------------------------------------------
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void mq32_attention_kernel(AttnParams p, int32_t qtiles) {
+  constexpr int kAccRow = 64 + 4;
+  __shared__ float s_ml[WAVES][2][16];
+  __shared__ __attribute__((aligned(16))) float s_acc[WAVES][16][kAccRow];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int g = lane >> 4, r = lane & 15;
+  const int h = blockIdx.x / qtiles, q0 = (blockIdx.x - h * qtiles) * 16, b = blockIdx.y;
+  const int len = min(max(p.lens[b], 0), p.max_len);
+  const int slot = p.slots ? p.slots[b] : b;
+  const int64_t base = (int64_t)slot * p.ss + (int64_t)(h / p.group) * p.sh;
+  const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint4*>(p.k + base), (short)0, (int)p.kv_bytes, kBufWord3);
+  const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint4*>(p.v + base), (short)0, (int)p.kv_bytes, kBufWord3);
+  const uint32_t row_bytes = (uint32_t)p.st * 16u;
+  auto load = [](__amdgpu_buffer_rsrc_t res, uint32_t off) __attribute__((always_inline)) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(res, off, 0, 0));
+  };
+  f32x4 q[4], kr[4], vr[4];
+  {
+    const int qi = min(q0 + r, p.qlen - 1);
+    const uint4* src = p.q + (int64_t)b * p.qsb + (int64_t)qi * p.qsq + (int64_t)h * p.qsh + 4 * g;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = __builtin_bit_cast(f32x4, src[i]);
+  }
+  auto load_k = [&](int t0) __attribute__((always_inline)) {
+    const uint32_t off = t0 + r < len ? (uint32_t)(t0 + r) * row_bytes + 64u * g : kBufOutOfRange;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) kr[i] = load(kres, off + 16u * i);
+  };
+  auto load_v = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = t0 + 4 * g + e;
+      vr[e] = load(vres, t < len ? (uint32_t)t * row_bytes + 16u * r : kBufOutOfRange);
+    }
+  };
+  f32x4 acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = kNegInf, l = 0.f;
+  int t0 = 16 * wave;
+  if (t0 < len) {
+    load_k(t0);
+    load_v(t0);
+  }
+  for (; t0 < len; t0 += 16 * WAVES) {
+    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[i][e], q[i][e], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[i][e + 1], q[i][e + 1], s1, 0, 0, 0);
+      }
+    load_k(t0 + 16 * WAVES);  // past the length: zeros, no memory read
+    float s[4], mx = m;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[e] = t0 + 4 * g + e < len ? (s0[e] + s1[e]) * p.scale_log2 : kNegInf;
+      mx = max_score(mx, s[e]);
+    }
+    mx = max_score(mx, xor_lane<16>(mx));
+    mx = max_score(mx, xor_lane<32>(mx));  // the query's, over the wave's keys so far
+    const float ref = mx == kNegInf ? 0.f : mx;
+    const float alpha = __builtin_amdgcn_exp2f(m - ref);
+    l *= alpha;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] *= alpha;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[e] = __builtin_amdgcn_exp2f(s[e] - ref);
+      l += s[e];
+    }
+    m = mx;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[e][i], s[e], acc[i], 0, 0, 0);
+    load_v(t0 + 16 * WAVES);
+  }
+  l += xor_lane<16>(l);
+  l += xor_lane<32>(l);
+  // Lane (g, r) holds query r, dims 16 g + 4 e + i in acc[i][e].
+  if (g == 0) {
+    s_ml[wave][0][r] = m;
+    s_ml[wave][1][r] = l;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    *reinterpret_cast<f32x4*>(&s_acc[wave][r][16 * g + 4 * e]) = f32x4{acc[0][e], acc[1][e], acc[2][e], acc[3][e]};
+  __syncthreads();
+  // 16 queries x 16 vectors of 4 dims.
+  for (int i = threadIdx.x; i < 256; i += 64 * WAVES) {
+    const int qi = i >> 4, c = i & 15;
+    if (q0 + qi >= p.qlen) continue;
+    float mm = s_ml[0][0][qi];
+    for (int w = 1; w < WAVES; ++w) mm = max_score(mm, s_ml[w][0][qi]);
+    const float ref = mm == kNegInf ? 0.f : mm;
+    float lt = 0.f;
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = __builtin_amdgcn_exp2f(s_ml[w][0][qi] - ref);
+      lt = fmaf(s_ml[w][1][qi], f, lt);
+      o += f * *reinterpret_cast<const f32x4*>(&s_acc[w][qi][4 * c]);
+    }
+    o *= lt > 0.f || lt != lt ? 1.f / lt : 0.f;
+    p.o[(int64_t)b * p.osb + (int64_t)(q0 + qi) * p.osq + (int64_t)h * p.osh + c] = __builtin_bit_cast(uint4, o);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Multi-query attention on the matrix cores (q_len >= 2, head_dim 64, fp16/bf16): the
 // cross-attention of a prompt, attention over encoder blocks, and a prompt's own causal
 // attention with its fused append (PROMPT).
@@ -2549,6 +2672,27 @@ void launch_mqt(int32_t dtype, const AttnParams& p, hipStream_t s) {
     launch_mqt_dt<SKV_F16, PAGED>(p, s);
 }
 
+// Whether fp32 attention of several queries takes the matrix cores: with enough query-key pairs that re-reading K and V per
+// query costs more than padding to 16 queries. Measured (us, one workgroup per query / matrix cores; batch x queries, heads,
+// keys): 1 x 4, 20, 1500 (120k pairs) 13.4 / 21.5; 4 x 4, 12, 700 (134k) 13.2 / 13.2; 8 x 2, 20, 1500 (480k) 42.9 / 30.3;
+// 20 x 10, 8, 400 (640k) 27.2 / 11.1; 50 x 4, 20, 1500 377 / 142; 1 x 1500, 20, 1500 1967 / 154.
+bool use_mq32(const AttnParams& p) {
+  return p.qlen >= 2 && (int64_t)p.batch * p.qlen * p.heads * p.max_len >= 200 * 1024;
+}
+
+void launch_mq32(const AttnParams& p, hipStream_t s) {
+  const int32_t qtiles = (int32_t)cdiv(p.qlen, 16);
+  const dim3 grid((uint32_t)(p.heads * qtiles), (uint32_t)p.batch);
+  const int64_t groups = (int64_t)p.heads * qtiles * p.batch;
+  // Few workgroups: more waves each share the keys.
+  if (groups <= 256 && p.max_len > 128)
+    hipLaunchKernelGGL((mq32_attention_kernel<16>), grid, dim3(1024), 0, s, p, qtiles);
+  else if (groups <= 512 && p.max_len > 64)
+    hipLaunchKernelGGL((mq32_attention_kernel<8>), grid, dim3(512), 0, s, p, qtiles);
+  else
+    hipLaunchKernelGGL((mq32_attention_kernel<4>), grid, dim3(256), 0, s, p, qtiles);
+}
+
 // Whether the 64-query kernel serves a multi-query launch: enough queries per row,
 // (row, head, 64 queries) workgroups for at least three quarters of the compute units
 // (it does not split keys across workgroups; below that the 16-query kernel, which
@@ -3020,6 +3164,11 @@ int skv_dense_attention(const void* q, int64_t q_stride_b, int64_t q_stride_q, i
       launch_mqt<false>(dtype, p, (hipStream_t)stream);
     else
       launch_mq<false>(dtype, p, (hipStream_t)stream);
+    return check_launch("skv_dense_attention");
+  }
+  if (dtype == SKV_F32 && head_dim == 64 && !is_prompt(p) && p.kv_bytes <= kBufLimit && p.st > 0 && batch <= 65535 &&
+      use_mq32(p)) {
+    launch_mq32(p, (hipStream_t)stream);
     return check_launch("skv_dense_attention");
   }
   rc = dispatch_attention<false>(dtype, head_dim, p, (hipStream_t)stream);
