@@ -715,6 +715,8 @@ def decode_linear_normed(x: torch.Tensor, stats: torch.Tensor, gamma: torch.Tens
     if ops is None:
         return None
     x2, m, n, k, code = ops
+    if stats.dtype != torch.float32 or stats.shape != (m, k // 16, 2) or not stats.is_contiguous() or not stats.is_cuda:
+        return None
     for t in (gamma, beta):
         if t.dtype != x.dtype or t.shape != (k,) or t.stride(0) != 1 or not t.is_cuda:
             return None

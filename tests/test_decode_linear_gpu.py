@@ -163,6 +163,7 @@ def test_fused_projection_refuses_what_it_does_not_take(cuda):
     s, st = native.decode_linear_residual(big, w, None, big)
     assert native.decode_linear_normed(s, st, b, b, 1e-5, w) is None  # past the decode batch
     assert native.decode_linear_normed(s[:8], st[:8], b[1:], b, 1e-5, w) is None
+    assert native.decode_linear_normed(s[:8], st[:7], b, b, 1e-5, w) is None
     nan = a.clone()
     nan[3, 7] = float("nan")  # reaches its own row only
     s, st = native.decode_linear_residual(nan, w, b, res)
