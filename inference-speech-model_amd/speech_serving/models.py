@@ -229,9 +229,10 @@ def _bucket_mask_lens(mask: torch.Tensor, rows: int, width: int, what: str) -> t
 
 
 def _hooked(mod: nn.Module) -> bool:
-    """Whether calling the module would run forward hooks (its own or global ones)."""
-    return bool(mod._forward_hooks or mod._forward_pre_hooks or nn.modules.module._global_forward_hooks or
-                nn.modules.module._global_forward_pre_hooks)
+    """Whether calling the module runs more than its class's forward: forward hooks (its own or global ones), or a
+    forward set on the instance."""
+    return bool(mod._forward_hooks or mod._forward_pre_hooks or "forward" in mod.__dict__ or
+                nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks)
 
 
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -251,6 +252,12 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] 
 
 def _plain(mod: nn.Module) -> bool:
     return type(mod) is nn.Linear and not _hooked(mod)
+
+
+def _plain_norm(mod: nn.Module) -> bool:
+    """Whether calling the module is nn.LayerNorm's own affine forward and nothing else."""
+    return isinstance(mod, nn.LayerNorm) and type(mod).forward is nn.LayerNorm.forward and not _hooked(mod) and \
+        mod.weight is not None and mod.bias is not None
 
 
 def proj(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
@@ -302,18 +309,16 @@ def mlp(seq: nn.Module, x: torch.Tensor) -> torch.Tensor:
 
 
 def add_norm(x: torch.Tensor, y: Union[torch.Tensor, native.Partials, None],
-             norm: nn.LayerNorm) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(s, norm(s)) for s = x + y (s = x when y is None): one native launch on the GPU (which also sums
-    the Partials of a split projection), the same two torch ops elsewhere."""
-    if x.is_cuda and norm.elementwise_affine and not _hooked(norm):
-        bias = norm.bias
-        if bias is not None:
-            if isinstance(y, native.Partials):
-                got = native.reduce_add_layernorm(y, x, norm.weight, bias, norm.eps)
-            else:
-                got = native.add_layernorm(x, y, norm.weight, bias, norm.eps, fallback=True)
-            if got is not None:
-                return got
+             norm: nn.Module) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(s, norm(s)) for s = x + y (s = x when y is None): one native launch for a LayerNorm on the GPU (which also
+    sums the Partials of a split projection), the same two torch ops for another norm and elsewhere."""
+    if x.is_cuda and _plain_norm(norm):
+        if isinstance(y, native.Partials):
+            got = native.reduce_add_layernorm(y, x, norm.weight, norm.bias, norm.eps)
+        else:
+            got = native.add_layernorm(x, y, norm.weight, norm.bias, norm.eps, fallback=True)
+        if got is not None:
+            return got
     s = x if y is None else x + _tensor(y)
     return s, norm(s)
 
@@ -348,8 +353,7 @@ class Residual:
     def normed_linear(self, norm: nn.Module, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                       gelu: bool = False) -> Optional[torch.Tensor]:
         """act(norm(x) @ weight.T (+ bias)) as one launch, or None."""
-        if self.stats is None or type(norm) is not nn.LayerNorm or norm.weight is None or norm.bias is None or \
-                _hooked(norm):
+        if self.stats is None or not _plain_norm(norm):
             return None
         return native.decode_linear_normed(self.x, self.stats, norm.weight, norm.bias, norm.eps, weight, bias, gelu)
 

@@ -1,0 +1,117 @@
+"""Decoder layers outside the usual form (replaced or wrapped modules, unusual operands) against float64 torch.
+
+The layers serve their usual modules and operands in fused native launches. Everything else has to reach the module a
+user put there, with the tensors that it would see in plain torch.
+"""
+import copy
+import types
+
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from speech_serving import models, native
+from speech_serving.models import CrossKV, DecoderLayer, PagedKV
+
+pytestmark = pytest.mark.gpu
+
+D, HEADS = 128, 2
+EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
+
+
+def _attend(q, k, v, causal, keep=None):
+    """softmax(q k^T / 8) v of q [B, S, H, 64] over k, v [B, H, T, 64], in float64; keep [B, T]."""
+    s = torch.matmul(q.transpose(1, 2), k.transpose(2, 3).contiguous()) / 8.0
+    if causal:
+        s = s.masked_fill(torch.ones(s.shape[-2:], device=s.device).triu(1 + s.shape[-1] - s.shape[-2]) > 0, -torch.inf)
+    if keep is not None:
+        s = s.masked_fill(~keep[:, None, None, :], -torch.inf)
+    return torch.matmul(torch.softmax(s, -1), v).transpose(1, 2)
+
+
+@torch.no_grad()
+def _reference(layer, x, cross=None, keep=None, cross_keep=None):
+    """(output, k, v) of the layer in float64, its modules called as they stand; cross: encoder states [B, T, D]."""
+    m = copy.deepcopy(layer).double()
+    x = x.double()
+    b, s, _ = x.shape
+    split = lambda t: t.view(t.shape[0], t.shape[1], m.num_heads, 64)  # noqa: E731
+    h = m.norm1(x)
+    q, k, v = (split(mod(h)) for mod in (m.self_attn_q, m.self_attn_k, m.self_attn_v))
+    k, v = k.transpose(1, 2), v.transpose(1, 2)
+    x = x + m.self_attn_out(_attend(q, k, v, m.is_decoder, keep).reshape(b, s, -1))
+    h = m.norm2(x)
+    if cross is not None:
+        ck, cv = (split(mod(cross.double())).transpose(1, 2) for mod in (m.cross_attn_k, m.cross_attn_v))
+        x = x + m.cross_attn_out(_attend(split(m.cross_attn_q(h)), ck, cv, False, cross_keep).reshape(b, s, -1))
+        h = m.norm3(x)
+    return x + m.mlp(h), k, v
+
+
+def _layer(dt=torch.float32, d=D, heads=HEADS, is_decoder=False, seed=0):
+    torch.manual_seed(seed)
+    layer = DecoderLayer(d, heads, 64, is_decoder=is_decoder)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.copy_(torch.randn_like(p) * (0.2 if p.dim() == 1 else p.shape[-1] ** -0.5) + (1.0 if p.dim() == 1 else 0.0))
+    return layer.to("cuda", dt)
+
+
+def _paged(layer, b, s, dt=torch.float32):
+    """An empty paged cache for b rows of s tokens."""
+    blocks = -(-s // 16)
+    pools = [torch.zeros(b * blocks, 16, layer.num_heads, 64, device="cuda", dtype=dt) for _ in range(2)]
+    tables = torch.arange(b * blocks, dtype=torch.int32, device="cuda").view(b, blocks)
+    return PagedKV([pools[0]], [pools[1]], tables, torch.full((b,), s, dtype=torch.int32, device="cuda"), blocks * 16)
+
+
+def _forms(layer, x):
+    """The layer's output over x by forward, and (causal layers) by forward_paged."""
+    with torch.no_grad():
+        out = [layer(x)[0]]
+        if layer.is_decoder:
+            y = layer.forward_paged(x, 0, _paged(layer, x.shape[0], x.shape[1], x.dtype), None)
+            out.append(y[0] + y[1])
+    return out
+
+
+def _close(got, want, what, rel=2e-6):
+    err = float((got.double() - want).norm() / want.norm())
+    assert got.shape == want.shape and err < rel, f"{what}: relative error {err:.2e}"
+
+
+class Doubled(nn.LayerNorm):
+    def forward(self, x):
+        return 2.0 * super().forward(x)
+
+
+class Renamed(nn.LayerNorm):
+    """LayerNorm under another name, its forward its own."""
+
+
+def _patched(norm):
+    norm.forward = types.MethodType(lambda self, x: 3.0 * F.layer_norm(x, (D,), self.weight, self.bias), norm)
+    return norm
+
+
+NORMS = {"subclass with its own forward": lambda: Doubled(D), "Identity": nn.Identity, "RMSNorm": lambda: nn.RMSNorm(D),
+         "no affine": lambda: nn.LayerNorm(D, elementwise_affine=False), "no bias": lambda: nn.LayerNorm(D, bias=False),
+         "subclass": lambda: Renamed(D), "forward set on the instance": lambda: _patched(nn.LayerNorm(D))}
+
+
+@pytest.mark.parametrize("kind", NORMS)
+@pytest.mark.parametrize("is_decoder", [False, True])
+def test_replaced_norm_is_the_one_that_runs(cuda, kind, is_decoder):
+    layer = _layer(is_decoder=is_decoder)
+    x = torch.randn(2, 20, D, device="cuda")
+    for name in ("norm1", "norm2", "norm3"):
+        setattr(layer, name, NORMS[kind]().to("cuda"))
+    want = _reference(layer, x)[0]
+    for got in _forms(layer, x):
+        _close(got, want, kind)
+    seen = []
+    for norm in (layer.norm1, layer.norm2):
+        norm.register_forward_hook(lambda mod, args, out: seen.append(mod))
+    _forms(layer, x)
+    assert seen == [layer.norm1, layer.norm2] * (1 + is_decoder)
