@@ -829,12 +829,10 @@ def reduce_add_layernorm(p: Partials, x: Optional[torch.Tensor], weight: Optiona
     x2 = None
     if x is not None:
         got = _layernorm_rows(x, x if weight is None else weight)
-        if got is None or x.dtype != p.dtype or x.shape != p.shape:
+        if got is None or x.dtype != p.dtype or x.shape != p.shape or x.get_device() != p.part.get_device():
             return None
         x2 = got[0]
-    if weight is not None and (weight.dtype != p.dtype or not weight.is_contiguous() or weight.numel() != h or
-                               weight.data_ptr() % 16 or bias.dtype != p.dtype or not bias.is_contiguous() or
-                               bias.numel() != h or bias.data_ptr() % 16):
+    if weight is not None and not (_norm_vector(weight, p.part, p.dtype, h) and _norm_vector(bias, p.part, p.dtype, h)):
         return None
     s = torch.empty(p.shape, dtype=p.dtype, device=p.part.device)
     norm = None if weight is None else torch.empty(p.shape, dtype=p.dtype, device=p.part.device)
@@ -867,6 +865,12 @@ def _layernorm_rows(x: torch.Tensor, weight: torch.Tensor):
     return x2, h, epl
 
 
+def _norm_vector(t: torch.Tensor, like: torch.Tensor, dtype: torch.dtype, h: int) -> bool:
+    """Whether t is a weight or bias that the LayerNorm kernels read: [h] of the dtype on like's GPU, 16-byte aligned."""
+    return t.dtype == dtype and t.numel() == h and t.is_contiguous() and t.data_ptr() % 16 == 0 and \
+        t.get_device() == like.get_device()
+
+
 def _add_layernorm_contiguous(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, bias: torch.Tensor,
                               eps: float) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
     """add_layernorm of contiguous tensors, the layers' case, with as little host work as it takes; None for any other
@@ -874,14 +878,14 @@ def _add_layernorm_contiguous(x: torch.Tensor, y: Optional[torch.Tensor], weight
     dt = x.dtype
     h = x.shape[-1]
     code = _DTYPE_CODE.get(dt)
-    if code is None or not x.is_cuda or h == 0 or h % 8 or h > 2048 or weight.dtype != dt or bias.dtype != dt or \
-            weight.shape != (h,) or bias.shape != (h,) or not weight.is_contiguous() or not bias.is_contiguous() or \
-            x.data_ptr() % 16:
+    if code is None or not x.is_cuda or h == 0 or h % 8 or h > 2048 or x.data_ptr() % 16 or \
+            not _norm_vector(weight, x, dt, h) or not _norm_vector(bias, x, dt, h):
         return None
     s = x
     yp = sp = None
     if y is not None:
-        if y.dtype != dt or y.shape != x.shape or not y.is_contiguous() or not y.is_cuda or y.data_ptr() % 16:
+        if y.dtype != dt or y.shape != x.shape or not y.is_contiguous() or y.data_ptr() % 16 or \
+                y.get_device() != x.get_device():
             return None
         s = torch.empty_like(x)
         yp, sp = y.data_ptr(), s.data_ptr()
@@ -897,27 +901,27 @@ def add_layernorm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tens
                   fallback: bool = False) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
     """(s, LayerNorm(s)) with s = x + y rounded to x's dtype (s = x when y is None).
 
-    x, y [..., hidden]; weight, bias [hidden]. sum_out may be x (in-place residual). An x the kernel
-    does not take (a CPU tensor, another dtype, a hidden size that is not a multiple of the 16-byte
+    x, y [..., hidden]; weight, bias [hidden]. sum_out may be x (in-place residual). Operands the kernel
+    does not take (on the CPU or another GPU, another dtype, a hidden size that is not a multiple of the 16-byte
     vector or above 512 of them, rows that are not 16-byte aligned, a weight or bias of another size)
-    raises RuntimeError, or with fallback=True returns None (the caller then runs torch's ops).
+    raise RuntimeError, or with fallback=True return None (the caller then runs torch's ops).
     """
     if sum_out is None and x.is_contiguous():
         got = _add_layernorm_contiguous(x, y, weight, bias, eps)
         if got is not None:
             return got
     got = _layernorm_rows(x, weight)
-    if got is not None and (not weight.is_contiguous() or weight.numel() != got[1] or bias.dtype != x.dtype or
-                            not bias.is_contiguous() or bias.numel() != got[1]):
-        got = None
+    y2 = None
+    if got is not None:
+        x2, h, epl = got
+        rows = x2.shape[0]
+        if not _norm_vector(weight, x, x.dtype, h) or not _norm_vector(bias, x, x.dtype, h):
+            got = None
     if got is None:
         if fallback:
             return None
         _gpu(x, "x")
-        raise RuntimeError("add_layernorm: unsupported dtype, hidden size, layout or weight/bias shape")
-    x2, h, epl = got
-    rows = x2.shape[0]
-    y2 = None
+        raise RuntimeError("add_layernorm: unsupported dtype, device, hidden size, layout or weight/bias shape")
     if y is not None:
         _gpu(y, "y")
         y2 = y.reshape(rows, h)

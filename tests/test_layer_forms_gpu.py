@@ -115,3 +115,38 @@ def test_replaced_norm_is_the_one_that_runs(cuda, kind, is_decoder):
         norm.register_forward_hook(lambda mod, args, out: seen.append(mod))
     _forms(layer, x)
     assert seen == [layer.norm1, layer.norm2] * (1 + is_decoder)
+
+
+def _offset(p, elements):
+    """The parameter's values at an address `elements` past a 16-byte line (a view into a flat buffer)."""
+    flat = torch.empty(p.numel() + 8, device=p.device, dtype=p.dtype)
+    view = flat[elements:elements + p.numel()].view(p.shape)
+    return nn.Parameter(view.copy_(p.detach()))
+
+
+@pytest.mark.parametrize("name", ["weight", "bias"])
+@pytest.mark.parametrize("is_decoder", [False, True])
+def test_norm_parameters_inside_a_flat_buffer(cuda, name, is_decoder):
+    layer = _layer(is_decoder=is_decoder)
+    x = torch.randn(2, 20, D, device="cuda")
+    want = _reference(layer, x)[0]
+    for norm in (layer.norm1, layer.norm2, layer.norm3):
+        setattr(norm, name, _offset(getattr(norm, name), 1))
+        assert getattr(norm, name).data_ptr() % 16 == 4
+    for got in _forms(layer, x):
+        _close(got, want, name)
+
+
+def test_norm_operands_on_another_device_are_refused(cuda):
+    x, w = torch.randn(8, D, device="cuda"), torch.ones(D, device="cuda")
+    for bad in ((x, None, w.cpu(), w), (x, None, w, w.cpu())):
+        assert native.add_layernorm(*bad, 1e-5, fallback=True) is None
+        with pytest.raises(RuntimeError, match="unsupported"):
+            native.add_layernorm(*bad, 1e-5)
+    part = native.Partials(torch.zeros(2, 8, D, device="cuda"), None, torch.Size((8, D)), torch.float32)
+    for bad in ((x, w.cpu(), w), (x, w, w.cpu())):
+        assert native.reduce_add_layernorm(part, *bad, 1e-5) is None
+    layer = _layer()
+    layer.norm2.weight = nn.Parameter(layer.norm2.weight.detach().cpu())
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        layer(x.view(2, 4, D))
