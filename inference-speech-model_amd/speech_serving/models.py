@@ -324,8 +324,8 @@ def add_norm(x: torch.Tensor, y: Union[torch.Tensor, native.Partials, None],
 
 
 def _sum_norm(x: torch.Tensor, y: Optional[torch.Tensor], norm: nn.Module) -> Tuple[torch.Tensor, torch.Tensor]:
-    """add_norm, in torch's own ops where x takes part in autograd."""
-    if x.requires_grad or (y is not None and y.requires_grad):
+    """add_norm, in torch's own ops where x takes part in autograd or y is to be broadcast."""
+    if x.requires_grad or (y is not None and (y.requires_grad or y.shape != x.shape)):
         s = x if y is None else x + y
         return s, norm(s)
     return add_norm(x, y, norm)

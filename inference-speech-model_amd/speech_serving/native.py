@@ -903,7 +903,7 @@ def add_layernorm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tens
 
     x, y [..., hidden]; weight, bias [hidden]. sum_out may be x (in-place residual). Operands the kernel
     does not take (on the CPU or another GPU, another dtype, a hidden size that is not a multiple of the 16-byte
-    vector or above 512 of them, rows that are not 16-byte aligned, a weight or bias of another size)
+    vector or above 512 of them, rows that are not 16-byte aligned, a y, weight or bias of another size)
     raise RuntimeError, or with fallback=True return None (the caller then runs torch's ops).
     """
     if sum_out is None and x.is_contiguous():
@@ -917,18 +917,20 @@ def add_layernorm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tens
         rows = x2.shape[0]
         if not _norm_vector(weight, x, x.dtype, h) or not _norm_vector(bias, x, x.dtype, h):
             got = None
+        elif y is not None:
+            if y.dtype != x.dtype or y.numel() != x.numel() or y.get_device() != x.get_device():
+                got = None
+            else:
+                y2 = y.reshape(rows, h)
+                if y2.stride(-1) != 1 or y2.data_ptr() % 16 or (rows > 1 and y2.stride(0) % epl):
+                    got = None
     if got is None:
         if fallback:
             return None
         _gpu(x, "x")
-        raise RuntimeError("add_layernorm: unsupported dtype, device, hidden size, layout or weight/bias shape")
-    if y is not None:
-        _gpu(y, "y")
-        y2 = y.reshape(rows, h)
-        if y2.dtype != x.dtype or y2.stride(-1) != 1 or y2.data_ptr() % 16:
-            raise RuntimeError("add_layernorm: y must match x's dtype with 16-byte rows")
-        if sum_out is None:
-            sum_out = torch.empty_like(x)
+        raise RuntimeError("add_layernorm: unsupported dtype, device, hidden size, layout or y/weight/bias shape")
+    if y is not None and sum_out is None:
+        sum_out = torch.empty_like(x)
     s2 = sum_out.reshape(rows, h) if sum_out is not None else None
     norm = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     many = rows > 1

@@ -137,9 +137,36 @@ def test_norm_parameters_inside_a_flat_buffer(cuda, name, is_decoder):
         _close(got, want, name)
 
 
+class Through(nn.Module):
+    """A projection whose result passes through f."""
+
+    def __init__(self, inner, f):
+        super().__init__()
+        self.inner, self.f = inner, f
+
+    def forward(self, x):
+        return self.f(self.inner(x))
+
+
+RESULTS = {"another dtype": lambda y: y.to(torch.bfloat16),
+           "broadcast over positions": lambda y: y.mean(1, keepdim=True),
+           "rows between 16-byte lines": lambda y: F.pad(y, (1, 0))[..., 1:],
+           "channels apart": lambda y: torch.stack((y, y), -1)[..., 0]}
+
+
+@pytest.mark.parametrize("kind", RESULTS)
+def test_projection_results_as_torch_would_add_them(cuda, kind):
+    layer = _layer()
+    layer.self_attn_out = Through(layer.self_attn_out, RESULTS[kind])
+    x = torch.randn(2, 20, D, device="cuda")
+    want = _reference(layer, x)[0]
+    # bfloat16 rounds the attention output once: 2^-9 of a term of the sum
+    _close(_forms(layer, x)[0], want, kind, 2.0 ** -9 if kind == "another dtype" else 2e-6)
+
+
 def test_norm_operands_on_another_device_are_refused(cuda):
     x, w = torch.randn(8, D, device="cuda"), torch.ones(D, device="cuda")
-    for bad in ((x, None, w.cpu(), w), (x, None, w, w.cpu())):
+    for bad in ((x, None, w.cpu(), w), (x, None, w, w.cpu()), (x, x.cpu(), w, w)):
         assert native.add_layernorm(*bad, 1e-5, fallback=True) is None
         with pytest.raises(RuntimeError, match="unsupported"):
             native.add_layernorm(*bad, 1e-5)
