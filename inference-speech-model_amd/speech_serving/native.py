@@ -930,8 +930,8 @@ def add_layernorm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tens
         _gpu(x, "x")
         raise RuntimeError("add_layernorm: unsupported dtype, device, hidden size, layout or y/weight/bias shape")
     if y is not None and sum_out is None:
-        sum_out = torch.empty_like(x)
-    s2 = sum_out.reshape(rows, h) if sum_out is not None else None
+        sum_out = torch.empty(x.shape, dtype=x.dtype, device=x.device)  # empty_like would keep permuted strides
+    s2 = sum_out.view(rows, h) if sum_out is not None else None  # the caller's memory, never a copy
     norm = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     many = rows > 1
     rc = lib().skv_add_layernorm(x2.data_ptr(), x2.stride(0) if many else h, _ptr(y2),

@@ -177,3 +177,16 @@ def test_norm_operands_on_another_device_are_refused(cuda):
     layer.norm2.weight = nn.Parameter(layer.norm2.weight.detach().cpu())
     with torch.no_grad(), pytest.raises(RuntimeError):
         layer(x.view(2, 4, D))
+
+
+@pytest.mark.parametrize("is_decoder", [False, True])
+def test_input_of_permuted_rows(cuda, is_decoder):
+    layer = _layer(is_decoder=is_decoder)
+    x = torch.randn(20, 3, D, device="cuda").transpose(0, 1)  # dense, positions outermost
+    want = _reference(layer, x)[0]
+    for got in _forms(layer, x):
+        _close(got, want, "permuted")
+    y, w, b = torch.randn(3, 20, D, device="cuda"), torch.randn(D, device="cuda"), torch.randn(D, device="cuda")
+    s, n = native.add_layernorm(x, y, w, b, 1e-5)
+    assert torch.equal(s, x + y)
+    _close(n, F.layer_norm((x + y).double(), (D,), w.double(), b.double(), 1e-5), "permuted norm")
