@@ -692,7 +692,7 @@ def decode_linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: Optional
         return None
     x2, m, n, k, code = ops
     r2 = res.reshape(m, n)
-    if n % 16 or r2.stride(1) != 1:
+    if n % 16 or r2.stride(1) != 1 or (m > 1 and r2.stride(0) < n):  # e.g. rows broadcast from one (stride 0)
         return None
     y = torch.empty(res.shape, dtype=x.dtype, device=x.device)
     stats = torch.empty((m, n // 16, 2), dtype=torch.float32, device=x.device)

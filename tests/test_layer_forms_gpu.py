@@ -190,3 +190,15 @@ def test_input_of_permuted_rows(cuda, is_decoder):
     s, n = native.add_layernorm(x, y, w, b, 1e-5)
     assert torch.equal(s, x + y)
     _close(n, F.layer_norm((x + y).double(), (D,), w.double(), b.double(), 1e-5), "permuted norm")
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_residual_rows_broadcast_from_one(cuda, dt):
+    layer = _layer(dt, 256, 4, is_decoder=True)
+    x = torch.randn(1, 1, 256, device="cuda").to(dt).expand(8, 1, 256)  # row stride 0
+    want = _reference(layer, x)[0]
+    y = layer.forward_paged(x, 0, _paged(layer, 8, 1, dt), None)
+    _close(y[0].double() + y[1].double(), want, "expanded residual", 2e-6 if dt == torch.float32 else 2 * EPS[dt])
+    a, w = torch.randn(8, 256, device="cuda").to(dt), layer.self_attn_out.weight
+    assert native.decode_linear_residual(a, w, None, x[:, 0]) is None
+    assert native.decode_linear_residual(a[:1], w, None, x[:1, 0]) is not None
