@@ -563,11 +563,14 @@ def _layer_step(layer: nn.Module, r: Residual, index: int, kv: PagedKV, cross: O
     return Residual(*layer.forward_paged(r.x, index, kv, cross, None if r.y is None else _tensor(r.y)))
 
 
-def _last_normed(r: Residual, last_only: bool, norm: nn.Module) -> torch.Tensor:
-    """norm of the stream (of its last position only, if last_only)."""
-    if last_only and r.x.shape[1] > 1:
-        r = Residual(r.x[:, -1:], None if r.y is None else _tensor(r.y)[:, -1:])
-    return r.normed(norm)
+def _last(r: Residual) -> Residual:
+    """The stream of the last position alone, [B, D]."""
+    y = r.y
+    if isinstance(y, native.Partials) and r.x.shape[1] == 1:
+        y = y.view(r.x.shape[0], r.x.shape[2])
+    elif y is not None:
+        y = _tensor(y)[:, -1]
+    return Residual(r.x[:, -1], y)
 
 
 # ---------------------------------------------------------------------------
@@ -653,8 +656,9 @@ class WhisperClassSpeechEncoderDecoderModel(nn.Module):
         r = Residual(self._embed(input_ids))
         for l, layer in enumerate(self.decoder_layers):
             r = _layer_step(layer, r, l, kv, cross)
-        h = _last_normed(r, last_only, self.decoder_norm)
-        return proj(self.lm_head, h[:, 0] if last_only else h)
+        if last_only:
+            r = _last(r)
+        return proj(self.lm_head, r.normed(self.decoder_norm))
 
     # -- decode step, reference signature (models.py:369-423) ----------------------------
     def decode_step(self, input_ids: torch.Tensor, past_key_values: Optional[Any] = None,
@@ -933,5 +937,7 @@ class StreamingMultiCodebookTTSModel(nn.Module):
         r = Residual(self.embeddings(input_codebooks))
         for l, layer in enumerate(self.layers):
             r = _layer_step(layer, r, l, kv, None)
-        logits = self.heads(_last_normed(r, last_only, self.norm))
+        if last_only and r.x.shape[1] > 1:
+            r = Residual(r.x[:, -1:], None if r.y is None else _tensor(r.y)[:, -1:])
+        logits = self.heads(r.normed(self.norm))
         return logits[:, 0] if last_only else logits

@@ -790,6 +790,9 @@ class Partials:
     def __init__(self, part: torch.Tensor, bias: Optional[torch.Tensor], shape: torch.Size, dtype: torch.dtype):
         self.part, self.bias, self.shape, self.dtype = part, bias, shape, dtype
 
+    def view(self, *shape: int) -> "Partials":
+        return Partials(self.part, self.bias, torch.Size(shape), self.dtype)
+
     def tensor(self) -> torch.Tensor:
         return reduce_add_layernorm(self, None, None, None, 0.0)[0]
 

@@ -202,3 +202,25 @@ def test_residual_rows_broadcast_from_one(cuda, dt):
     a, w = torch.randn(8, 256, device="cuda").to(dt), layer.self_attn_out.weight
     assert native.decode_linear_residual(a, w, None, x[:, 0]) is None
     assert native.decode_linear_residual(a[:1], w, None, x[:1, 0]) is not None
+
+
+@pytest.mark.parametrize("d,heads", [(128, 2), (512, 8), (1024, 16)])  # fc2 by torch's library, unsplit, and in partials
+@pytest.mark.parametrize("s", [1, 5])
+def test_final_norm_is_called_with_the_last_position(cuda, d, heads, s):
+    """decode_step_paged calls the final norm and the LM head on [B, D] rows, and logits agree with every position's."""
+    torch.manual_seed(3)
+    m = models.WhisperClassSpeechEncoderDecoderModel(0, 2, heads, d, 80, 264, 64).to("cuda")
+    ids = torch.randint(0, 264, (3, s), device="cuda")
+    pools = [_paged(m.decoder_layers[0], 3, s) for _ in range(2)]
+    kv = PagedKV([p.k_pools[0] for p in pools], [p.v_pools[0] for p in pools], pools[0].block_tables,
+                 pools[0].ctx_lens, pools[0].max_ctx)
+    shapes = []
+    with torch.no_grad():
+        every = m.decode_step_paged(ids, kv, last_only=False)
+        plain = m.decode_step_paged(ids, kv)
+        for mod in (m.decoder_norm, m.lm_head):
+            mod.register_forward_hook(lambda mod, args, out: shapes.append(tuple(args[0].shape)))
+        hooked = m.decode_step_paged(ids, kv)
+    assert shapes == [(3, d), (3, d)] and plain.shape == (3, 264)
+    for got in (plain, hooked):
+        _close(got, every[:, -1].double(), "last position")
