@@ -554,11 +554,13 @@ class DecoderLayer(nn.Module):
         return x + mlp(self.mlp, h), new_past, new_cross
 
 
+_FORWARD_PAGED = DecoderLayer.forward_paged
+
+
 def _layer_step(layer: nn.Module, r: Residual, index: int, kv: PagedKV, cross: Optional[CrossKV]) -> Residual:
     """layer.forward_paged on the stream, its MLP output added or handed on as the projection left it; a layer whose
-    forward_paged is overridden is called through it, with tensors."""
-    if getattr(type(layer), "forward_paged", None) is DecoderLayer.forward_paged and \
-            "forward_paged" not in layer.__dict__:
+    forward_paged is overridden (or wrapped, on the class or the instance) is called through it, with tensors."""
+    if getattr(type(layer), "forward_paged", None) is _FORWARD_PAGED and "forward_paged" not in layer.__dict__:
         return layer._step_paged(r, index, kv, cross, add=True)
     return Residual(*layer.forward_paged(r.x, index, kv, cross, None if r.y is None else _tensor(r.y)))
 

@@ -224,3 +224,31 @@ def test_final_norm_is_called_with_the_last_position(cuda, d, heads, s):
     assert shapes == [(3, d), (3, d)] and plain.shape == (3, 264)
     for got in (plain, hooked):
         _close(got, every[:, -1].double(), "last position")
+
+
+@pytest.mark.parametrize("where", ["class", "subclass", "instance"])
+def test_wrapped_forward_paged_is_called(cuda, where, monkeypatch):
+    torch.manual_seed(4)
+    m = models.WhisperClassSpeechEncoderDecoderModel(0, 2, 8, 512, 80, 264, 64).to("cuda")
+    ids = torch.randint(0, 264, (3, 1), device="cuda")
+    pools = [_paged(m.decoder_layers[0], 3, 1) for _ in range(2)]
+    kv = PagedKV([p.k_pools[0] for p in pools], [p.v_pools[0] for p in pools], pools[0].block_tables,
+                 pools[0].ctx_lens, pools[0].max_ctx)
+    seen, original = [], DecoderLayer.forward_paged
+
+    def wrapper(self, x, layer, kv, cross, pending=None):
+        seen.append((layer, torch.is_tensor(x), pending is None or torch.is_tensor(pending)))
+        return original(self, x, layer, kv, cross, pending)
+
+    with torch.no_grad():
+        want = m.decode_step_paged(ids, kv)
+        if where == "class":
+            monkeypatch.setattr(DecoderLayer, "forward_paged", wrapper)
+        for layer in m.decoder_layers:
+            if where == "subclass":
+                layer.__class__ = type("Wrapped", (DecoderLayer,), {"forward_paged": wrapper})
+            elif where == "instance":
+                layer.forward_paged = types.MethodType(wrapper, layer)
+        got = m.decode_step_paged(ids, kv)
+    assert seen == [(0, True, True), (1, True, True)]
+    _close(got, want.double(), where)
