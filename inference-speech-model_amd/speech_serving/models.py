@@ -38,6 +38,7 @@ from typing import Any, List, Optional, Sequence, Tuple, Union
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import native
 
@@ -323,12 +324,21 @@ def add_norm(x: torch.Tensor, y: Union[torch.Tensor, native.Partials, None],
     return s, norm(s)
 
 
-def _sum_norm(x: torch.Tensor, y: Optional[torch.Tensor], norm: nn.Module) -> Tuple[torch.Tensor, torch.Tensor]:
-    """add_norm, in torch's own ops where x takes part in autograd or y is to be broadcast."""
-    if x.requires_grad or (y is not None and (y.requires_grad or y.shape != x.shape)):
+def _sum_norm(x: torch.Tensor, y: Optional[torch.Tensor], norm: nn.Module,
+              ends: bool = True) -> Tuple[torch.Tensor, torch.Tensor]:
+    """add_norm, in torch's own ops where y is to be broadcast or a derivative is taken: x or y take part in autograd or
+    carry a tangent, or the norm's parameters may get gradients (ends False: what takes the norm passes them on; the
+    native projections do not)."""
+    if x.requires_grad or _tangent(x) or \
+            (y is not None and (y.requires_grad or y.shape != x.shape or _tangent(y))) or \
+            (not ends and torch.is_grad_enabled() and any(p.requires_grad for p in norm.parameters())):
         s = x if y is None else x + y
         return s, norm(s)
     return add_norm(x, y, norm)
+
+
+def _tangent(x: torch.Tensor) -> bool:
+    return forward_ad.unpack_dual(x).tangent is not None
 
 
 class Residual:
@@ -528,7 +538,9 @@ class DecoderLayer(nn.Module):
         attn = native.dense_attention(q, kk, vv, lens, t, self.scale, causal=self.is_decoder and s > 1)
         new_cross = None
         used = encoder_hidden_states is not None or encoder_past_kv is not None
-        x, h = _sum_norm(x, proj(self.self_attn_out, attn.reshape(b, s, hd)), self.norm2)
+        parts = _mlp_parts(self.mlp, x)
+        ends = parts is not None and _plain(parts[0])
+        x, h = _sum_norm(x, proj(self.self_attn_out, attn.reshape(b, s, hd)), self.norm2, used or ends)
         if used:
             if encoder_past_kv is not None:
                 ck, cv = encoder_past_kv
@@ -550,7 +562,7 @@ class DecoderLayer(nn.Module):
                 ck, cv = ck.expand(b, -1, -1, -1), cv.expand(b, -1, -1, -1)
             cq = proj(self.cross_attn_q, h).view(b, s, self.num_heads, self.head_dim)
             c = native.dense_attention(cq, ck, cv, clens, te, self.scale)
-            x, h = _sum_norm(x, proj(self.cross_attn_out, c.reshape(b, s, hd)), self.norm3)
+            x, h = _sum_norm(x, proj(self.cross_attn_out, c.reshape(b, s, hd)), self.norm3, ends)
         return x + mlp(self.mlp, h), new_past, new_cross
 
 

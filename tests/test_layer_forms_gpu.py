@@ -252,3 +252,51 @@ def test_wrapped_forward_paged_is_called(cuda, where, monkeypatch):
         got = m.decode_step_paged(ids, kv)
     assert seen == [(0, True, True), (1, True, True)]
     _close(got, want.double(), where)
+
+
+class Plain(nn.Module):
+    """An MLP of torch's own ops."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, x):
+        for mod in self.inner:
+            x = mod(x)
+        return x
+
+
+@pytest.mark.parametrize("cross", [False, True])
+def test_gradients_reach_the_norm_ahead_of_a_torch_mlp(cuda, cross):
+    """Attention ends a graph here; what follows it in torch's ops passes gradients on to the norm's parameters."""
+    layer = _layer()
+    layer.mlp = Plain(layer.mlp)
+    x, enc = torch.randn(2, 20, D, device="cuda"), torch.randn(2, 9, D, device="cuda")
+    g = torch.randn(2, 20, D, device="cuda")
+    norm = layer.norm3 if cross else layer.norm2
+    out = layer(x, encoder_hidden_states=enc if cross else None)[0]
+    out.backward(g)
+    m = copy.deepcopy(layer).double()
+    m.zero_grad()
+    taken = []
+    (m.norm3 if cross else m.norm2).register_forward_pre_hook(lambda mod, args: taken.append(args[0]))
+    want = _reference(m, x, enc if cross else None)[0]
+    _close(out.detach(), want, "output")
+    s = taken[0]
+    ref = m.norm3 if cross else m.norm2
+    (s + m.mlp(ref(s))).backward(g.double())
+    for name in ("weight", "bias"):
+        _close(getattr(norm, name).grad, getattr(ref, name).grad, name, 1e-5)
+
+
+def test_tangents_pass_the_residual_adds(cuda):
+    layer = _layer()
+    layer.mlp = Plain(layer.mlp)
+    x, t = torch.randn(2, 20, D, device="cuda"), torch.randn(2, 20, D, device="cuda")
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        out = layer(torch.autograd.forward_ad.make_dual(x, t))[0]
+        got = torch.autograd.forward_ad.unpack_dual(out)
+        assert got.tangent is not None and got.tangent.shape == x.shape
+        primal = got.primal.clone()
+    _close(primal, _reference(layer, x)[0], "primal")
