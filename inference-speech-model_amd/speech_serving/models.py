@@ -238,10 +238,10 @@ def _hooked(mod: nn.Module) -> bool:
 
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
             gelu: bool = False) -> torch.Tensor:
-    """x @ weight.T (+ bias), then the erf GELU when gelu: a decode batch in one skv_decode_linear launch, more rows
-    with GELU in one skv_rows_linear launch, other shapes through skv_linear (a hipBLASLt plan cached per shape) and
-    torch's GELU."""
-    y = native.decode_linear(x, weight, bias, gelu)
+    """x @ weight.T (+ bias), then the erf GELU when gelu: a decode batch in one skv_decode_linear launch where that is
+    the faster way, more rows with GELU in one skv_rows_linear launch, other shapes through skv_linear (a hipBLASLt
+    plan cached per shape) and torch's GELU."""
+    y = native.decode_linear(x, weight, bias, gelu) if _decode_pays(x, weight, gelu) else None
     if y is None and gelu and x.numel() > native.DECODE_ROWS * x.shape[-1]:
         y = native.rows_linear(x, weight, bias, gelu=True)
     if y is None:
@@ -249,6 +249,16 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] 
         if gelu:
             y = F.gelu(y)
     return y
+
+
+def _decode_pays(x: torch.Tensor, weight: torch.Tensor, gelu: bool = False) -> bool:
+    k = x.shape[-1]
+    return k > 0 and native.decode_pays(x.numel() // k, weight.shape[0], k, x.dtype == torch.float32, gelu)
+
+
+def _partials(fc2: nn.Module, h: torch.Tensor) -> Optional[native.Partials]:
+    """fc2(h) in partial sums, where its contraction is split and that is the faster way."""
+    return native.decode_partials(h, fc2.weight, fc2.bias) if _decode_pays(h, fc2.weight) else None
 
 
 def _plain(mod: nn.Module) -> bool:
@@ -294,7 +304,7 @@ def _mlp(seq: nn.Module, x: torch.Tensor) -> Union[torch.Tensor, native.Partials
 
 def _mlp_out(fc2: nn.Module, h: torch.Tensor) -> Union[torch.Tensor, native.Partials]:
     if _plain(fc2):
-        y = native.decode_partials(h, fc2.weight, fc2.bias)
+        y = _partials(fc2, h)
         if y is not None:
             return y
     return proj(fc2, h)
@@ -501,7 +511,7 @@ class DecoderLayer(nn.Module):
         fc2 = parts[2]
         if not add or not _plain(fc2):
             return Residual(r.x, _mlp_out(fc2, h))
-        y = native.decode_partials(h, fc2.weight, fc2.bias)
+        y = _partials(fc2, h)
         return r.add(fc2, h) if y is None else Residual(r.x, y)
 
     # -- contiguous API of the reference (models.py:110-208) ---------------------

@@ -644,6 +644,33 @@ def decode_batch(x: torch.Tensor, n: int) -> bool:
     return size <= MAX_DECODE_ROWS * k and size * n <= (k << (18 if wide else 20)) and k <= (1024 if wide else 2048)
 
 
+def decode_pays(rows: int, n: int, k: int, wide: bool, gelu: bool = False) -> bool:
+    """Whether the library's own projection (skv_decode_linear; partials and their sum for rows past 6 KiB) is faster than
+    hipBLASLt (and, with gelu, a GELU launch) for a decode batch. wide: fp32.
+
+    The own kernel reads its x rows again in every workgroup and is made for one workgroup per compute unit, so it loses
+    where many outputs (an LM head) or many products make several rounds of workgroups. Own / hipBLASLt (us):
+    - 16-bit, to 2^30 products and 2^21 outputs, rows counted in whole tiles past 64: 128 x 8192 x 1024 10.6 / 12.8,
+      64 x 16384 x 1024 12.8 / 13.5; 96 x 8192 x 1280 11.6 / 11.0, 128 x 16384 x 1024 20.6 / 14.7, 128 x 25600 x 256
+      11.5 / 9.0, 64 x 51864 x 1280 44.7 / 32.6; in partials 64 x 2048 x 8192 17.3 / 26.6, 128 x 2048 x 8192 29.8 / 25.4.
+    - fp32, to 4096 outputs a row, or 2^28 products and 2^24 weights: 128 x 4096 x 1024 15.9 / 19.8, 64 x 8192 x 512
+      10.0 / 10.2, 16 x 25600 x 512 17.2 / 17.3; 64 x 8192 x 1024 17.7 / 14.5, 16 x 16384 x 1024 21.4 / 18.9.
+    - fp32 rows past 4 KiB leave one workgroup per unit: 64 x 3840 x 1280 12.6 / 14.7, 96 x 1280 x 1280 7.1 / 7.6,
+      with GELU 32 x 5120 x 1280 13.2 / 13.9; 80 x 3840 x 1280 21.4 / 15.5, 128 x 1280 x 1536 12.1 / 10.4, with GELU
+      64 x 5120 x 1280 22.7 / 18.9. In partials 64 rows, or 2^28 products: 64 x 1280 x 5120 21.6 / 35.3; 128 x 768 x 3072
+      18.1 / 15.3, 96 x 1280 x 5120 30.4 / 24.5."""
+    if not wide:
+        return rows * n <= 1 << 21 and (rows if rows <= 64 else -(-rows // 64) * 64) * n * k <= 1 << 30
+    work = rows * n * k
+    if k <= 1024:
+        return (n <= 4096 or work <= 1 << 28) and n * k < 1 << 24
+    if k > 1536:
+        return rows <= 64 or work <= 1 << 28
+    if rows > 64:
+        return -(-rows // 32) * -(-n // 32) <= 128
+    return n <= 4096 or (gelu and rows <= 32)
+
+
 def _proj_operands(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], max_rows: int):
     """(x as [m, k] rows, m, n, k, dtype code) of a decode projection, or None when the batch, the types or the
     layouts are not those skv_decode_linear takes (its own checks decide about sizes and alignment)."""
@@ -668,7 +695,8 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
                   gelu: bool = False) -> Optional[torch.Tensor]:
     """act(x @ weight.T (+ bias)) of a decode batch (or a short prompt batch) in one launch on the matrix cores, summed
     in fp32 and rounded once; gelu applies the erf GELU to the fp32 result. None for a call skv_decode_linear does
-    not take (the caller runs linear()). Reference: speech_serving/models.py:127-207."""
+    not take (the caller runs linear()); whether it is the faster way is decode_pays' to say. Reference:
+    speech_serving/models.py:127-207."""
     ops = _proj_operands(x, weight, bias, MAX_DECODE_ROWS) if decode_batch(x, weight.shape[0]) else None
     if ops is None:
         return None
@@ -804,7 +832,7 @@ def _decode_splits(k: int, code: int) -> int:
 
 def decode_partials(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[Partials]:
     """x @ weight.T (+ bias) as Partials when the projection's contraction is split, else None (a call that
-    decode_linear or linear takes)."""
+    decode_linear or linear takes). Whether it is the faster way is decode_pays' to say."""
     ops = _proj_operands(x, weight, bias, DECODE_ROWS)
     if ops is None:
         return None

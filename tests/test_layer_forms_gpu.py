@@ -300,3 +300,17 @@ def test_tangents_pass_the_residual_adds(cuda):
         assert got.tangent is not None and got.tangent.shape == x.shape
         primal = got.primal.clone()
     _close(primal, _reference(layer, x)[0], "primal")
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [51200, 51864])
+def test_lm_head_of_a_vocabulary_the_decode_kernel_takes(cuda, dt, n):
+    """proj over the rows around the crossover to the library, by whichever path serves them."""
+    head = nn.Linear(384, n, bias=False).to("cuda", dt)
+    for m in (1, 17, 40, 41, 64, 128):
+        x = torch.randn(m, 384, device="cuda").to(dt)
+        with torch.no_grad():
+            got = models.proj(head, x).double()
+            want = x.double() @ head.weight.double().t()
+            bound = 384 * 2.0 ** -24 * (x.double().abs() @ head.weight.double().abs().t())
+        assert bool(((got - want).abs() <= EPS[dt] * want.abs() + bound + 1e-30).all()), m
