@@ -551,29 +551,6 @@ void launch_argmax(int vecs, int32_t rows, hipStream_t s, const char* logits, in
   }
 }
 
-// The fp32 values of one 16-byte vector.
-template <int DT> __device__ __forceinline__ void unpack16(const uint4& v, float* f);
-template <> __device__ __forceinline__ void unpack16<SKV_F32>(const uint4& v, float* f) {
-  f[0] = __uint_as_float(v.x), f[1] = __uint_as_float(v.y), f[2] = __uint_as_float(v.z), f[3] = __uint_as_float(v.w);
-}
-template <> __device__ __forceinline__ void unpack16<SKV_F16>(const uint4& v, float* f) {
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const half2v h = __builtin_bit_cast(half2v, w[i]);
-    f[2 * i] = (float)h.x;
-    f[2 * i + 1] = (float)h.y;
-  }
-}
-template <> __device__ __forceinline__ void unpack16<SKV_BF16>(const uint4& v, float* f) {
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = bf16_lo(w[i]);
-    f[2 * i + 1] = bf16_hi(w[i]);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Multi-codebook embedding sum: out[r] = T_0[c_r0] + T_1[c_r1] + ... with every
 // partial sum rounded to the tensor dtype, i.e. the bits of a sequential

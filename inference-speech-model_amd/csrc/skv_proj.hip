@@ -366,9 +366,9 @@ __global__ __launch_bounds__(64 * WAVES) void proj_kernel(
 //   y   = sum_s part[s] + bias   (fp32, splits in order), or the given tensor
 //   sum = x + y rounded to the tensor type
 //   norm = LayerNorm(sum) * gamma + beta, fp32 statistics in two passes over registers
-// One workgroup per row, 4 elements per thread: a launch is its floor, one round of loads and two reductions, so
-// the elements per lane decide (1280 bf16 elements, 64 rows: 2.73 us; with one wave per row, 24 elements per lane,
-// 4.26 us; 256 elements 2.01 / 2.57 us, 1608 rows of 1280 5.5 / 5.9 us).
+// One workgroup per row, 4 elements per thread: for few rows a launch is its floor, one round of loads and two
+// reductions, so the elements per lane decide (64 x 1280 fp32 3.1 us, one wave per row 3.8). Many rows and short ones take
+// add_norm_rows_kernel.
 // ---------------------------------------------------------------------------
 constexpr int kMaxNormVecs = 512;  // 16-byte vectors of a row
 
@@ -432,7 +432,116 @@ __global__ __launch_bounds__(1024) void add_norm_kernel(AddNormParams p) {
   if (in) store_quad<DT>(p.norm, row * p.ldn + 4 * c, d * rstd * gm + bt);
 }
 
+// The same without partials, one wave per row (4 rows per workgroup, VPL 16-byte vectors per lane). Many rows are bound by
+// memory, and there its wide accesses and the want of a barrier count: 12000 x 1280 bf16 22.3 us (5.5 TB/s; one
+// workgroup per row 37.4), without the add 12.3 (22.9), fp16 22.4 (38.0).
+template <int DT, int VPL>
+__global__ __launch_bounds__(256) void add_norm_rows_kernel(AddNormParams p, int32_t rows) {
+  constexpr int EPL = Elt<DT>::EPL;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;  // uniform over the wave
+  const int vecs = p.quads * 4 / EPL;
+  const uint4* x = reinterpret_cast<const uint4*>(p.x) + row * (p.ldx / EPL);
+  uint4 raw[VPL], gv[VPL], bv[VPL];
+  // Every load up front (x, y, gamma, beta): one memory round trip per row.
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int c = lane + 64 * j;
+    raw[j] = gv[j] = bv[j] = make_uint4(0u, 0u, 0u, 0u);
+    if (c < vecs) {
+      raw[j] = x[c];
+      gv[j] = reinterpret_cast<const uint4*>(p.gamma)[c];
+      bv[j] = reinterpret_cast<const uint4*>(p.beta)[c];
+    }
+  }
+  auto pack = [](const float* f) __attribute__((always_inline)) {
+    if constexpr (DT == SKV_BF16) {  // fp16: the packed form is the slower one here (64 x 1280 3.9 us against 3.4)
+      return make_uint4(pack2<DT>(f[0], f[1]), pack2<DT>(f[2], f[3]), pack2<DT>(f[4], f[5]), pack2<DT>(f[6], f[7]));
+    } else {
+      return pack16<DT>(f);
+    }
+  };
+  if (p.y) {
+    const uint4* y = reinterpret_cast<const uint4*>(p.y) + row * (p.ldy / EPL);
+    uint4 ry[VPL];
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      ry[j] = make_uint4(0u, 0u, 0u, 0u);
+      if (lane + 64 * j < vecs) ry[j] = y[lane + 64 * j];
+    }
+    uint4* sum = reinterpret_cast<uint4*>(p.sum) + (p.sum ? row * (p.lds / EPL) : 0);
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      float a[EPL], b[EPL];
+      unpack16<DT>(raw[j], a);
+      unpack16<DT>(ry[j], b);
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) a[e] += b[e];
+      raw[j] = pack(a);  // rounded to the tensor type, like the stored sum
+      if (p.sum && lane + 64 * j < vecs) sum[lane + 64 * j] = raw[j];
+    }
+  }
+  float v[VPL][EPL], s = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    unpack16<DT>(raw[j], v[j]);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) s += v[j][e];
+  }
+  const float mean = group_sum<64>(s) * p.inv_n;
+  float q = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      v[j][e] -= mean;
+      if (lane + 64 * j < vecs) q = fmaf(v[j][e], v[j][e], q);
+    }
+  }
+  const float rstd = rsqrtf(group_sum<64>(q) * p.inv_n + p.eps);
+  uint4* norm = reinterpret_cast<uint4*>(p.norm) + row * (p.ldn / EPL);
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    if (lane + 64 * j >= vecs) continue;
+    float g[EPL], b[EPL];
+    unpack16<DT>(gv[j], g);
+    unpack16<DT>(bv[j], b);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) g[e] = v[j][e] * rstd * g[e] + b[e];
+    norm[lane + 64 * j] = pack(g);
+  }
+}
+
+// One wave per row but for long rows (past 2 KiB) of a decode batch or a short prompt, where the elements per lane decide.
+// Wave / workgroup per row (us, with the add): bf16 64 x 1024 3.0 / 3.1, 64 x 1280 3.5 / 3.3, 256 x 2048 4.1 / 4.0,
+// 512 x 1280 4.0 / 4.1, 800 x 2048 5.4 / 5.9, 3000 x 1280 7.9 / 9.9; fp32 64 x 512 2.8 / 2.7, 64 x 1280 3.8 / 3.1,
+// 800 x 1280 5.6 / 5.3, 1500 x 1280 7.6 / 7.9, without the add 3000 x 1280 7.3 / 8.2.
+bool norm_by_waves(int rows, int vecs, int32_t dtype) { return vecs <= 128 || rows >= (dtype == SKV_F32 ? 1024 : 512); }
+
+template <int DT>
+void launch_add_norm_rows(const AddNormParams& p, int rows, int vecs, hipStream_t s) {
+  const dim3 grid((uint32_t)cdiv(rows, 4)), block(256);
+  switch (cdiv(vecs, 64)) {
+    case 1: hipLaunchKernelGGL((add_norm_rows_kernel<DT, 1>), grid, block, 0, s, p, rows); break;
+    case 2: hipLaunchKernelGGL((add_norm_rows_kernel<DT, 2>), grid, block, 0, s, p, rows); break;
+    case 3: hipLaunchKernelGGL((add_norm_rows_kernel<DT, 3>), grid, block, 0, s, p, rows); break;
+    case 4: hipLaunchKernelGGL((add_norm_rows_kernel<DT, 4>), grid, block, 0, s, p, rows); break;
+    case 5: hipLaunchKernelGGL((add_norm_rows_kernel<DT, 5>), grid, block, 0, s, p, rows); break;
+    default: hipLaunchKernelGGL((add_norm_rows_kernel<DT, 8>), grid, block, 0, s, p, rows); break;
+  }
+}
+
 void launch_add_norm(const AddNormParams& p, int rows, int32_t dtype, hipStream_t s) {
+  const int vecs = p.quads / (dtype == SKV_F32 ? 1 : 2);
+  if (!p.part && norm_by_waves(rows, vecs, dtype)) {
+    switch (dtype) {
+      case SKV_F32: launch_add_norm_rows<SKV_F32>(p, rows, vecs, s); break;
+      case SKV_F16: launch_add_norm_rows<SKV_F16>(p, rows, vecs, s); break;
+      default: launch_add_norm_rows<SKV_BF16>(p, rows, vecs, s); break;
+    }
+    return;
+  }
   const dim3 grid((uint32_t)rows), block((uint32_t)cdiv(p.quads, 64) * 64);
   switch (dtype) {
     case SKV_F32: hipLaunchKernelGGL((add_norm_kernel<SKV_F32>), grid, block, 0, s, p); break;

@@ -85,3 +85,24 @@ def test_add_layernorm_in_graph_replays(cuda):
         torch.cuda.synchronize()
         assert torch.equal(s, x + y)
         check_norm(n.cpu(), ln64((x + y).cpu(), w.cpu(), b.cpu(), 1e-5), dt, f"replay {it}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [8, 520, 1032, 1280, 2048])
+def test_many_rows_and_strided_rows(cuda, dtype, hidden):
+    """Row counts around the change from a workgroup to a wave per row (512; fp32 1024) and of a partial last workgroup,
+    over rows inside wider ones; hidden sizes of one to eight vectors per lane."""
+    gen = torch.Generator(device="cuda").manual_seed(hidden)
+    for rows in (3, 511, 513, 1023, 1025, 6001):
+        wide = torch.full((2, rows, hidden + 16), float("nan"), device="cuda", dtype=dtype)
+        x, y = wide[:, :, 8:8 + hidden]
+        for t in (x, y):
+            t.copy_(torch.randn(rows, hidden, generator=gen, device="cuda") * 3 + 0.5)
+        w, b = ((1 + 0.2 * torch.randn(hidden, generator=gen, device="cuda")).to(dtype) for _ in range(2))
+        want_s = x + y
+        s, n = native.add_layernorm(x, y, w, b, 1e-5)
+        assert torch.equal(s, want_s), f"rows={rows}"
+        check_norm(n, ln64(want_s, w, b, 1e-5), dtype, f"rows={rows}")
+        _, n = native.add_layernorm(x, None, w, b, 1e-5)
+        check_norm(n, ln64(x, w, b, 1e-5), dtype, f"no add rows={rows}")
+        assert bool(torch.isnan(wide[:, :, :8]).all()) and bool(torch.isnan(wide[:, :, 8 + hidden:]).all())
