@@ -45,12 +45,18 @@ __device__ __forceinline__ f32x4 mfma_16x16x32(const uint4& a, const uint4& b, c
   }
 }
 
-// The erf GELU x Phi(x), Phi(-|x|) = t 2^(P(t) - x^2 / 2 log2 e) with t = 1 / (1 + |x| / sqrt 8) and P a Chebyshev fit of
-// degree 9 to log2(erfcx(|x| / sqrt 2) / 2t) over |x| <= 13.5. Relative error below 1.3e-6 for x > -5 and 7.3e-6 for
-// x > -13, absolute below 3.9e-7, where x / 2 (1 + erff(x / sqrt 2)) loses the negative tail to cancellation (4.7e-2
-// relative, 4.5e-7 absolute). About 20 operations without a branch; erff takes more than twice that, which was a third of
-// a 1500 x 5120 x 1280 projection (36 us with it, 26 without GELU).
+// The erf GELU x Phi(x) of an fp32 value. fp32 results take x / 2 (1 + erff(x / sqrt 2)), which is exact to the last bits near
+// zero, where most pre-activations lie (largest relative error on |x| < 0.1 1.2e-7; the fit below 4.2e-7).
+//
+// 16-bit results, of 2^-9 and 2^-12, take Phi(-|x|) = t 2^(P(t) - x^2 / 2 log2 e) with t = 1 / (1 + |x| / sqrt 8): the form
+// of the Chebyshev fit to erfc of Press et al. (Numerical Recipes, erfcc) in base 2, P fitted here, of degree 9, to
+// log2(erfcx(|x| / sqrt 2) / 2t) over |x| <= 13.5. Relative error below 1.3e-6 for x > -5 and 7.3e-6 for
+// x > -13, absolute below 3.9e-7. About 20 operations without a branch; erff takes more than twice that, which was a third
+// of a 1500 x 5120 x 1280 projection (36 us with it, 26 without GELU); a decode batch's fp32 launch pays 0.25 us for it
+// (4 x 1536 x 384 3.7 us against 3.4 with the fit, 64 x 3072 x 768 8.3 against 8.1).
+template <int DT>
 __device__ __forceinline__ float gelu(float x) {
+  if constexpr (DT == SKV_F32) return 0.5f * x * (1.f + erff(x * 0.70710678119f));
   const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(x), 0.35355339059f, 1.f));
   float p = fmaf(0.203332633f, t, -0.950718999f);
   p = fmaf(p, t, 1.59427726f);

@@ -206,7 +206,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmParams p) {
     if (p.bias) add16<DT>(v, p.bias + 2 * col);
     if (p.act) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = gelu(v[e]);
+      for (int e = 0; e < 8; ++e) v[e] = gelu<DT>(v[e]);
     }
     if (p.res) add16<DT>(v, p.res + 2 * ((int64_t)row * p.ldr + col));
     char* d;

@@ -343,7 +343,7 @@ __global__ __launch_bounds__(64 * WAVES) void proj_kernel(
     v += widen<DT>(bias[o]);
     if (p.act) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = gelu(v[e]);
+      for (int e = 0; e < 4; ++e) v[e] = gelu<DT>(v[e]);
     }
     v += widen<DT>(res[o]);
     v = round_quad<DT>(v);

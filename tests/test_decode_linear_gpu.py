@@ -170,3 +170,17 @@ def test_fused_projection_refuses_what_it_does_not_take(cuda):
     y = native.decode_linear_normed(s, st, b, b, 1e-5, w)
     bad = torch.isnan(y).any(dim=1)
     assert bool(bad[3]) and int(bad.sum()) == 1
+
+
+def test_fp32_gelu_is_as_exact_as_torch(cuda):
+    """Over identity weights the products are x itself, so the GELU's own error shows: on every interval at most torch's
+    (x / 2 (1 + erff), to a percent for another erff), which is the smallest near zero."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    w = torch.eye(128, device="cuda")
+    for lo, hi in ((0.0, 0.1), (0.1, 0.3), (0.3, 1.0), (1.0, 2.0), (2.0, 4.0), (4.0, 9.0)):
+        for sign in (-1.0, 1.0):
+            x = sign * (lo + (hi - lo) * torch.rand(128, 128, generator=g, device="cuda"))
+            want = F.gelu(x.double())
+            err, ref = ((y.double() - want) / want.abs().clamp_min(1e-30) for y in (native.decode_linear(x, w, gelu=True), F.gelu(x)))
+            assert float(err.norm()) <= 1.01 * float(ref.norm()), (sign * lo, sign * hi)
+            assert float(err.abs().max()) <= 1.01 * float(ref.abs().max()), (sign * lo, sign * hi)
