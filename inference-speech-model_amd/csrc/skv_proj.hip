@@ -78,8 +78,10 @@ __device__ __forceinline__ uint4 load_cached(__amdgpu_buffer_rsrc_t r, uint32_t 
 }
 
 // The elements of a 16-byte vector of x, normalised and rounded to the dtype: (x - mean) * rstd * gamma + beta.
-// st: mean and rstd, for 16-bit rows -mean * rstd and rstd (one operation less; the fp32 rounding it adds is
-// |mean / std| 2^-24 against the 2^-9 or 2^-12 of the result).
+// st: mean and rstd, for 16-bit rows -mean * rstd and rstd (one operation less; with the subtraction first 64 x 1280 x 1280
+// takes 6.1 us instead of 5.9). The rounding this adds is no larger than the mean's own in fp32: over identity weights the
+// error against float64 is that of the LayerNorm launch to 0.1 %, for a mean of 8 to 475 times the spread (fp16, mean 400:
+// 2.080e-4 / 2.078e-4, torch in fp32 2.081e-4; mean 64 2.075e-4 in all three).
 template <int DT>
 __device__ __forceinline__ uint4 norm16(const uint4& x, const uint4& gamma, const uint4& beta, float2 st) {
   const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, gw[4] = {gamma.x, gamma.y, gamma.z, gamma.w};

@@ -184,3 +184,20 @@ def test_fp32_gelu_is_as_exact_as_torch(cuda):
             err, ref = ((y.double() - want) / want.abs().clamp_min(1e-30) for y in (native.decode_linear(x, w, gelu=True), F.gelu(x)))
             assert float(err.norm()) <= 1.01 * float(ref.norm()), (sign * lo, sign * hi)
             assert float(err.abs().max()) <= 1.01 * float(ref.abs().max()), (sign * lo, sign * hi)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+def test_normed_projection_is_as_exact_as_the_layernorm_launch(cuda, dt):
+    """Over identity weights, for rows whose mean is up to 400 times their spread: the error against float64 is at most a
+    percent above that of the LayerNorm launch (in fp32, where the mean's rounding is all there is, a tenth)."""
+    for mean, d in ((0, 512), (8, 512), (64, 256), (64, 1024), (400, 1024)):
+        g = torch.Generator(device="cuda").manual_seed(mean + d)
+        res = (torch.randn(64, d, generator=g, device="cuda") + mean).to(dt)
+        zeros, one, eye = (t.to("cuda", dt) for t in (torch.zeros(64, 256), torch.ones(d), torch.eye(d)))
+        s, stats = native.decode_linear_residual(zeros, zeros.new_zeros(d, 256), None, res)
+        assert torch.equal(s, res)
+        want = F.layer_norm(s.double(), (d,), eps=1e-5)
+        y = native.decode_linear_normed(s, stats, one, zeros.new_zeros(d), 1e-5, eye)
+        n = native.add_layernorm(s, None, one, zeros.new_zeros(d), 1e-5)[1]
+        err, ref = (float((t.double() - want).norm()) for t in (y, n))
+        assert err <= (1.1 if dt == torch.float32 else 1.01) * ref, (mean, d, err, ref)
