@@ -1538,8 +1538,8 @@ __global__ __launch_bounds__(64 * WAVES) void mq32_attention_kernel(AttnParams p
 // Online softmax per query (base 2), the max over a 32-key step reduced across
 // the 4 lane groups. P enters its product with V in the input dtype: fp16 rounds
 // it once (the row sums then add the rounded values, so the weights stay a convex
-// combination); bf16, and prompts in either dtype, add the product of the rounded
-// remainder, which keeps the weights to ~16 bits (fp16 22).
+// combination); bf16 adds the product of the rounded remainder, which keeps the weights
+// to ~16 bits, and prompts in either dtype one more (kPOperands).
 // The waves merge through LDS; a split row writes per-query partials that
 // merge_kernel combines.
 // ---------------------------------------------------------------------------
@@ -1638,6 +1638,32 @@ constexpr int kMqQueries = 16;  // queries per tile (the MFMA's N)
 // almost every step.
 constexpr float kLazyMaxLog2 = 8.f;
 
+// Operands that carry the softmax weights P into their product with V: a rounded head, then rounded remainders of what the
+// ones before it hold. Prompts keep P to all 24 bits, as the one-query kernel has it: three operands, of fp16 with P
+// kPromptScale times the weight, so that the remainders stay clear of fp16's subnormals (P below 2^15). Attention over
+// encoder keys takes two of bf16 and one of fp16, as the kernels' comments say.
+// With one operand less (bf16 16 bits, fp16 22) sums whose values cancel came out 1.5 to 2 and 1.0 to 1.25 times as far from
+// float64 as the one-query kernel's; now both are its equals (bf16, 201 tokens 5.6e-8 -> 2.6e-8 of sum |p v|, one query
+// 2.6e-8; fp16, 4 tokens 4.4e-8 -> 3.5e-8 / 3.5e-8). It costs little: 20 heads, bf16, 8 x 201 16.8 -> 17.3 us, 8 x 64
+// 6.4 -> 6.45, 128 x 4 6.25 -> 6.3.
+template <int DT, bool PROMPT>
+constexpr int kPOperands = PROMPT ? 3 : DT == SKV_BF16 ? 2 : 1;
+template <int DT, bool PROMPT>
+constexpr float kPromptScale = PROMPT && DT == SKV_F16 ? 128.f : 1.f;
+
+// The next operand of the 8 weights, which keep what it leaves.
+template <int DT>
+__device__ __forceinline__ uint4 next_operand(float (&p)[8]) {
+  uint32_t w[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    w[k] = pack2<DT>(p[2 * k], p[2 * k + 1]);
+    p[2 * k] -= lo16<DT>(w[k]);
+    p[2 * k + 1] -= hi16<DT>(w[k]);
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // 3 waves per SIMD: the register budget that holds the next step's loads in flight without
 // spilling (4 spills and halves the rate; 2 is no faster).
 // PAGED: K/V come from the block pools through the row's table (power-of-two block size of
@@ -1647,7 +1673,8 @@ template <int DT, bool PAGED, bool PROMPT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3))) void
 mq_attention_kernel(AttnParams p, int32_t qtiles) {
   static_assert(WAVES == 4 || WAVES == 1, "each wave finalises 4 / WAVES of the 16-dim blocks");
-  constexpr bool kSplitP = DT == SKV_BF16 || PROMPT;  // P as a rounded head plus the rounded remainder
+  constexpr int kOps = kPOperands<DT, PROMPT>;  // operands of P
+  constexpr float kScale = kPromptScale<DT, PROMPT>;
   constexpr int D = 64;
   constexpr int PSTRIDE = D + kPartPad;
   __shared__ float s_m[WAVES][kMqQueries];
@@ -1874,29 +1901,26 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
       l *= alpha;
       m = mn;
     }
-    // P^T operand. fp16 rounds P once (unit roundoff 2^-11) and the row sums add the rounded
-    // values; bf16 (2^-8) splits P into a rounded head and the rounded remainder, two products
-    // with the same V^T, so the weights keep ~16 bits and the sums use P itself.
-    uint32_t pw[4], pr[4];
+    // P^T operands. One fp16 operand rounds P (unit roundoff 2^-11) and the row sums add the rounded values; more
+    // operands hold P to 16 bits or more (kPOperands), all multiply the same V^T, and the sums use P itself.
+    float ps[8];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float p0 = __builtin_amdgcn_exp2f(sv[2 * k] - ref);
-      const float p1 = __builtin_amdgcn_exp2f(sv[2 * k + 1] - ref);
-      const uint32_t w = pack2<DT>(p0, p1);
-      pw[k] = w;
-      if constexpr (kSplitP) {
-        pr[k] = pack2<DT>(p0 - lo16<DT>(w), p1 - hi16<DT>(w));
-        l += p0 + p1;
-      } else {
-        l += lo16<DT>(w) + hi16<DT>(w);
-      }
+    for (int k = 0; k < 8; ++k) ps[k] = __builtin_amdgcn_exp2f(sv[k] - ref) * kScale;
+    if constexpr (kOps > 1) {
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) l += ps[k] + ps[k + 1];
     }
-    const uint4 pt = make_uint4(pw[0], pw[1], pw[2], pw[3]);
-    const uint4 prt = make_uint4(pr[0], pr[1], pr[2], pr[3]);
 #pragma unroll
-    for (int db = 0; db < 4; ++db) {
-      acc[db] = mfma_16x16x32<DT>(vt[db], pt, acc[db]);
-      if constexpr (kSplitP) acc[db] = mfma_16x16x32<DT>(vt[db], prt, acc[db]);
+    for (int o = 0; o < kOps; ++o) {
+      const uint4 pt = next_operand<DT>(ps);
+      if constexpr (kOps == 1) {
+        l += lo16<DT>(pt.x) + hi16<DT>(pt.x);
+        l += lo16<DT>(pt.y) + hi16<DT>(pt.y);
+        l += lo16<DT>(pt.z) + hi16<DT>(pt.z);
+        l += lo16<DT>(pt.w) + hi16<DT>(pt.w);
+      }
+#pragma unroll
+      for (int db = 0; db < 4; ++db) acc[db] = mfma_16x16x32<DT>(vt[db], pt, acc[db]);
     }
   };
   // Software pipeline: the next step's loads are in flight while this step computes.
@@ -1972,8 +1996,8 @@ mq_attention_kernel(AttnParams p, int32_t qtiles) {
               (uint16_t)pack2<DT>(l1 > 0.f ? a1 * (1.f / l1) : (l1 == 0.f ? 0.f : l1), 0.f);
         } else {
           float* rec = p.part + ((((int64_t)b * p.qlen + qs) * p.heads + h) * p.nchunk_max + chunk) * PSTRIDE;
-          rec[kPartPad + lane] = a1;
-          if (lane == 0) *reinterpret_cast<float2*>(rec) = make_float2(m1, l1);
+          rec[kPartPad + lane] = a1 * kScale;  // as the chunks of finite sums have it
+          if (lane == 0) *reinterpret_cast<float2*>(rec) = make_float2(m1, l1 * kScale);
         }
       }
       return;
@@ -2025,7 +2049,8 @@ __global__ __launch_bounds__(64 * kWaves * kMqtParts) __attribute__((amdgpu_wave
 mqt_attention_kernel(AttnParams p) {
   static_assert(kWaves * kMqQueries == kMqtQueries, "mqt_attention_kernel: 16 queries per wave");
   static_assert(kMqtParts == 2, "mqt_attention_kernel: the end-of-kernel merge is written for two parts");
-  constexpr bool kSplitP = DT == SKV_BF16 || PROMPT;  // P as a rounded head plus the rounded remainder
+  constexpr int kOps = kPOperands<DT, PROMPT>;  // operands of P
+  constexpr float kScale = kPromptScale<DT, PROMPT>;
   constexpr int D = 64;
   constexpr int STEP = 32;                       // keys per compute half-step
   constexpr int LSTEP = 64;                      // keys per staged step, 16 per wave
@@ -2211,7 +2236,7 @@ mqt_attention_kernel(AttnParams p) {
   // fp16 sums P on the matrix cores: a product with an operand of ones gives every lane
   // its query's sum over the step's 32 keys (the rounded weights, as the PV product
   // uses them). bf16 sums the unrounded weights on the VALU: its P is two operands.
-  constexpr bool kOnesSum = !kSplitP;
+  constexpr bool kOnesSum = kOps == 1;
   f32x4 l4 = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint4 ones = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);
 
@@ -2276,28 +2301,22 @@ mqt_attention_kernel(AttnParams p) {
         l *= alpha;
       m = mn;
     }
-    // P^T operand, as in mq_attention_kernel: fp16 rounds P once and sums the rounded
-    // values; bf16 adds the product of the rounded remainder.
-    uint32_t pw[4], pr[4];
+    // P^T operands, as in mq_attention_kernel.
+    float ps[8];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float p0 = __builtin_amdgcn_exp2f(fmaf(sv[2 * k], p.scale_log2, -ref));
-      const float p1 = __builtin_amdgcn_exp2f(fmaf(sv[2 * k + 1], p.scale_log2, -ref));
-      const uint32_t w = pack2<DT>(p0, p1);
-      pw[k] = w;
-      if constexpr (kSplitP) {
-        pr[k] = pack2<DT>(p0 - lo16<DT>(w), p1 - hi16<DT>(w));
-        l += p0 + p1;
-      }
-    }
-    const uint4 pt = make_uint4(pw[0], pw[1], pw[2], pw[3]);
-    const uint4 prt = make_uint4(pr[0], pr[1], pr[2], pr[3]);
+    for (int k = 0; k < 8; ++k) ps[k] = __builtin_amdgcn_exp2f(fmaf(sv[k], p.scale_log2, -ref)) * kScale;
+    if constexpr (!kOnesSum) {
 #pragma unroll
-    for (int db = 0; db < 4; ++db) {
-      acc[db] = mfma_16x16x32<DT>(vt[db], pt, acc[db]);
-      if constexpr (kSplitP) acc[db] = mfma_16x16x32<DT>(vt[db], prt, acc[db]);
+      for (int k = 0; k < 8; k += 2) l += ps[k] + ps[k + 1];
     }
-    if constexpr (kOnesSum) l4 = mfma_16x16x32<DT>(ones, pt, l4);
+    if constexpr (PROMPT) __builtin_amdgcn_sched_barrier(0);  // the scores' registers are free before the operands' are taken: no spills
+#pragma unroll
+    for (int o = 0; o < kOps; ++o) {
+      const uint4 pt = next_operand<DT>(ps);
+#pragma unroll
+      for (int db = 0; db < 4; ++db) acc[db] = mfma_16x16x32<DT>(vt[db], pt, acc[db]);
+      if constexpr (kOnesSum) l4 = mfma_16x16x32<DT>(ones, pt, l4);
+    }
   };
 
   // Step st's loads live in register slot st % 2 from their issue (one step ahead)
@@ -2591,14 +2610,14 @@ int bind_workspace(AttnParams& p, const char* who, int32_t d, void* ws, int64_t 
 bool is_prompt(const AttnParams& p) { return p.causal || p.kn; }
 
 // Prompts of at most this many keys take one wave per (row, head, 16 queries): one or two steps of keys leave nothing
-// for four waves to share, and four times the workgroups are resident (bf16 20 heads, 128 x 4 tokens 6.0 us, with four
+// for four waves to share, and four times the workgroups are resident (bf16 20 heads, 128 x 4 tokens 6.3 us, with four
 // waves 14.2; 32 x 32 tokens 8.0 / 9.9 us, 8 x 32 6.5 / 5.5 us).
 constexpr int kShortPrompt = 32;
 
 // Whether a prompt's queries go to the matrix-core kernels rather than one workgroup per (query, head): when those
 // would be four per compute unit or more, or have many keys each. Below that the launch is its floor and one
 // query's chain is shorter. Measured (us, one workgroup per query / matrix cores; bf16, fused append):
-//   20 heads: 8 x 4 tokens 4.2 / 4.2, 8 x 16 7.0 / 5.0, 8 x 64 21.6 / 6.2, 8 x 201 84.6 / 16.6, 128 x 4 18.8 / 6.0,
+//   20 heads: 8 x 4 tokens 4.2 / 4.2, 8 x 16 7.0 / 5.0, 8 x 64 21.6 / 6.4, 8 x 201 84.6 / 17.3, 128 x 4 18.8 / 6.3,
 //   128 x 32 133 / 21, 1 x 32 4.6 / 5.0; 4 heads: 1 x 64 4.7 / 5.5, 1 x 201 10.0 / 5.4, 32 x 8 4.5 / 4.4;
 //   after 200-3000 cached keys, 20 heads: 1 x 2 (400) 5.5 / 8.0, 8 x 2 (200) 6.9 / 7.7, 64 x 2 (200) 23.4 / 20.8,
 //   1 x 16 (3000) 27.5 / 17.8.
