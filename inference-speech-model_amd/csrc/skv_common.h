@@ -16,6 +16,8 @@ int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
 // Bytes per element of a dtype code; 0 if unknown.
 int elt_bytes(int32_t dtype);
+// Compute units of the current device (256, this GPU's, when the query fails), cached per device.
+int compute_units();
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }

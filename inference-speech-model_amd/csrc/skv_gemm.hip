@@ -13,8 +13,6 @@
 // workgroups starting at different k (no change); 192 x 128 tiles for every shape (38 against 26 us at 1500 x 5120).
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-
 #include "skv_common.h"
 #include "skv_device.h"
 #include "speech_kv.h"
@@ -220,17 +218,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmParams p) {
     *reinterpret_cast<uint4*>(d) =
         make_uint4(pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3]), pack2<DT>(v[4], v[5]), pack2<DT>(v[6], v[7]));
   }
-}
-
-int compute_units() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n > 0) return n;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
-  cache[dev].store(n, std::memory_order_relaxed);
-  return n;
 }
 
 // Tiles in units of 64 x 64, and their measured time for one step of 64 elements (us) with a workgroup per compute unit.

@@ -56,6 +56,17 @@ int check_launch(const char* what) {
   return SKV_OK;
 }
 
+int compute_units() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+  cache[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
+
 int elt_bytes(int32_t dtype) {
   switch (dtype) {
     case SKV_F32: return 4;
@@ -2480,22 +2491,6 @@ int32_t paged_chunk(int32_t rows, int32_t heads, int32_t kv_heads, int32_t d, in
 
 bool supported_d(int32_t d) { return d == 16 || d == 32 || d == 64 || d == 128; }
 
-// Compute units of the current device (0 when the query fails), cached per device.
-int device_cu_count() {
-  constexpr int kMaxDevices = 64;
-  static std::atomic<int> cache[kMaxDevices];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
-  if (dev < kMaxDevices) {
-    const int c = cache[dev].load(std::memory_order_relaxed);
-    if (c > 0) return c;
-  }
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
-  if (dev < kMaxDevices && n > 0) cache[dev].store(n, std::memory_order_relaxed);
-  return n;
-}
-
 template <int DT, int D, bool PAGED>
 void launch_attention(const AttnParams& p, hipStream_t stream) {
   const int64_t rh = (int64_t)p.batch * p.qlen * p.heads;
@@ -2580,8 +2575,8 @@ int prepare_attention(AttnParams& p, const char* who, const void* q, int64_t qsb
   p.nchunk_max = nchunk_max;
   p.grid3d = (int64_t)batch * q_len <= 65535;
   const int64_t items = (int64_t)batch * q_len * heads;
-  const int cus = device_cu_count();
-  p.snake = p.grid3d && nchunk_max == 1 && heads >= 2 && items * heads < ((int64_t)1 << 32) && cus > 0 &&
+  const int cus = compute_units();
+  p.snake = p.grid3d && nchunk_max == 1 && heads >= 2 && items * heads < ((int64_t)1 << 32) &&
             (cus & (cus - 1)) == 0;
   if (p.snake) {
     p.cu_shift = __builtin_ctz((unsigned)cus);
@@ -2698,7 +2693,7 @@ void launch_mq32(const AttnParams& p, hipStream_t s) {
 // unscaled scores).
 bool use_mqt(const AttnParams& p) {
   return p.qlen >= kMqtQueries && p.scale_log2 > 0.f &&
-         4 * (int64_t)p.batch * p.heads * cdiv(p.qlen, kMqtQueries) >= 3 * (int64_t)device_cu_count() &&
+         4 * (int64_t)p.batch * p.heads * cdiv(p.qlen, kMqtQueries) >= 3 * (int64_t)compute_units() &&
          (int64_t)p.heads * cdiv(p.qlen, kMqtQueries) <= 0x7fffffff;
 }
 

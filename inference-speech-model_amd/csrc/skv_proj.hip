@@ -21,8 +21,6 @@
 // workgroups (3.5 us alone, but the sum in the next launch takes the gain back: 7.45 / 7.46 us for the pair).
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-
 #include "skv_common.h"
 #include "skv_device.h"
 #include "speech_kv.h"
@@ -571,18 +569,6 @@ struct ProjShape {
   int mi, ni, waves, rounds;
   bool one_each;  // at most one workgroup per compute unit
 };
-
-// Compute units of the current device (256 when the query fails).
-int compute_units() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n > 0) return n;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
-  cache[dev].store(n, std::memory_order_relaxed);
-  return n;
-}
 
 int proj_splits(int64_t chunks) { return chunks <= kMaxSplitChunks ? 1 : (int)cdiv(chunks, kMaxChunks); }
 

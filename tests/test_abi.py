@@ -205,3 +205,25 @@ def test_library_was_built_from_this_tree():
     got = native.library_digest(native.lib())
     assert len(got) == 16 and got in native.expected_digests()
     assert f"src:{got}" in native.version()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_decode_batch_is_the_librarys_own_rule(dtype):
+    """native.decode_batch, asked before a projection's operands are prepared, against what skv_decode_linear answers at
+    each boundary: taken (then the null x is EINVAL) or SKV_EUNSUPPORTED."""
+    import torch
+
+    lib, dt = native.lib(), getattr(torch, dtype)
+    code, wide = native._DTYPE_CODE[dt], dtype == "float32"
+    limit = 1 << (18 if wide else 20)
+    taken = 0
+    for k in (512, 1024, 1028 if wide else 1032, 2048, 2056):
+        if wide and k > 1536:
+            continue  # split: partials
+        for m in (0, 1, 127, 128, 129, 256, 511, 512, 513):
+            for n in {4, limit // 512, limit // 512 + 4, limit // 256, limit // 256 + 4, 20480}:
+                rc = lib.skv_decode_linear(None, k, FAKE, k, None, 0, FAKE, n, m, n, k, code, None)
+                assert rc in ((0,) if m == 0 else (-1, native.SKV_EUNSUPPORTED)), (m, n, k)
+                assert native.decode_batch(torch.empty(m, k, dtype=dt, device="meta"), n) == (rc != native.SKV_EUNSUPPORTED), (m, n, k)
+                taken += rc == -1
+    assert taken > 20
