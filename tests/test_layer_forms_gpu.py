@@ -314,3 +314,34 @@ def test_lm_head_of_a_vocabulary_the_decode_kernel_takes(cuda, dt, n):
             want = x.double() @ head.weight.double().t()
             bound = 384 * 2.0 ** -24 * (x.double().abs() @ head.weight.double().abs().t())
         assert bool(((got - want).abs() <= EPS[dt] * want.abs() + bound + 1e-30).all()), m
+
+
+# rows past the decode batch: q/k/v by head, GELU in the epilogue, adds and norms in one launch (16-bit); fp32 attention of
+# several queries on the matrix cores (2 x 300 queries of 4 heads over 300 keys are past its bound)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("b,s", [(1, 150), (3, 97), (2, 300)])
+@pytest.mark.parametrize("is_decoder,form", [(False, "plain"), (False, "masked"), (False, "cross"), (True, "plain"),
+                                             (True, "cross"), (True, "cross masked")])
+def test_forward_of_many_rows(cuda, dt, b, s, is_decoder, form):
+    """DecoderLayer.forward over prompts and frames: output, returned K/V and cross K/V against float64."""
+    d, heads, te = 256, 4, 110
+    layer = _layer(dt, d, heads, is_decoder)
+    x = torch.randn(b, s, d, device="cuda").to(dt)
+    enc = torch.randn(b, te, d, device="cuda").to(dt) if "cross" in form else None
+    keep = cross_keep = None
+    if form == "masked":
+        keep = torch.arange(s, device="cuda")[None] < torch.randint(1, s + 1, (b, 1), device="cuda")
+        keep[0, ::3] = False  # not a prefix
+        keep[:, 1] = True
+    if form == "cross masked":
+        cross_keep = torch.arange(te, device="cuda")[None] < torch.randint(1, te + 1, (b, 1), device="cuda")
+    with torch.no_grad():
+        y, (k, v), cross = layer(x, encoder_hidden_states=enc,
+                                 attention_mask=None if keep is None else keep.long(),
+                                 encoder_attention_mask=None if cross_keep is None else cross_keep.long())
+    want, wk, wv = _reference(layer, x, enc, keep, cross_keep)
+    rel = 2e-6 if dt == torch.float32 else 2 * EPS[dt]  # a rounding of each of the layer's tensors, as root mean square
+    assert k.shape == (b, heads, s, 64)
+    for got, ref, what in ((y, want, "output"), (k, wk, "k"), (v, wv, "v")):
+        _close(got, ref, f"{form} {what}", rel)
+    assert (cross is None) == (enc is None)
