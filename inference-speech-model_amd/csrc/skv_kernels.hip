@@ -2664,11 +2664,15 @@ void launch_mqt(int32_t dtype, const AttnParams& p, hipStream_t s) {
 }
 
 // Whether fp32 attention of several queries takes the matrix cores: with enough query-key pairs that re-reading K and V per
-// query costs more than padding to 16 queries. Measured (us, one workgroup per query / matrix cores; batch x queries, heads,
-// keys): 1 x 4, 20, 1500 (120k pairs) 13.4 / 21.5; 4 x 4, 12, 700 (134k) 13.2 / 13.2; 8 x 2, 20, 1500 (480k) 42.9 / 30.3;
-// 20 x 10, 8, 400 (640k) 27.2 / 11.1; 50 x 4, 20, 1500 377 / 142; 1 x 1500, 20, 1500 1967 / 154.
+// query costs more than padding to 16 queries, and than a workgroup's chain over long rows (t keys in 16 waves: about 22 us
+// for 1500). Measured (us, one workgroup per query / matrix cores; batch x queries, heads, keys):
+//   1 x 4, 20, 1500 (117 Ki pairs) 13.4 / 21.5; 4 x 4, 12, 700 (131 Ki) 13.2 / 13.2; 12 x 4, 20, 220 (206 Ki) 15.2 / 9.0;
+//   1 x 300, 4, 300 (351 Ki) 11.6 / 9.4; 20 x 10, 8, 400 (625 Ki) 27.2 / 11.1; 1 x 1500, 20, 1500 1967 / 154;
+//   past 320 keys 1 x 100, 4, 600 (234 Ki) 11.0 / 12.7, 1 x 64, 8, 600 (300 Ki) 11.3 / 12.9, 1 x 100, 6, 600 (351 Ki) 18.6 /
+//   12.9, 1 x 32, 8, 1500 (375 Ki) 15.0 / 21.9, 4 x 4, 16, 1500 (375 Ki) 21.2 / 24.8, 1 x 16, 20, 1500 (468 Ki) 24.1 / 21.8.
 bool use_mq32(const AttnParams& p) {
-  return p.qlen >= 2 && (int64_t)p.batch * p.qlen * p.heads * p.max_len >= 200 * 1024;
+  const int64_t pairs = (int64_t)p.batch * p.qlen * p.heads * p.max_len;
+  return p.qlen >= 2 && pairs >= 200 * 1024 + (p.max_len > 320 ? 180 * (int64_t)p.max_len : 0);
 }
 
 void launch_mq32(const AttnParams& p, hipStream_t s) {
