@@ -2615,11 +2615,11 @@ constexpr int kShortPrompt = 32;
 //   20 heads: 8 x 4 tokens 4.2 / 4.2, 8 x 16 7.0 / 5.0, 8 x 64 21.6 / 6.4, 8 x 201 84.6 / 17.3, 128 x 4 18.8 / 6.3,
 //   128 x 32 133 / 21, 1 x 32 4.6 / 5.0; 4 heads: 1 x 64 4.7 / 5.5, 1 x 201 10.0 / 5.4, 32 x 8 4.5 / 4.4;
 //   after 200-3000 cached keys, 20 heads: 1 x 2 (400) 5.5 / 8.0, 8 x 2 (200) 6.9 / 7.7, 64 x 2 (200) 23.4 / 20.8,
-//   1 x 16 (3000) 27.5 / 17.8.
+//   1 x 16 (3000) 27.5 / 17.8; of 300 keys 2 x 16, 8 heads (75 Ki query-key pairs) 5.6 / 7.9, 12 heads (112 Ki) 7.1 / 8.6.
 bool prompt_on_mfma(const AttnParams& p) {
   const int64_t items = (int64_t)p.batch * p.qlen * p.heads, work = items * p.max_len;
-  return (items >= 1024 && (p.qlen >= 4 || p.max_len <= kShortPrompt)) || (p.qlen >= 16 && work >= 40 * 1024) ||
-         work >= 160 * 1024;
+  return (items >= 1024 && (p.qlen >= 4 || p.max_len <= kShortPrompt)) ||
+         (p.qlen >= 16 && p.max_len <= 4 * p.qlen && work >= 40 * 1024) || work >= 160 * 1024;
 }
 
 // The multi-query matrix-core attention (fp16/bf16, head_dim 64) and, for split rows, the merge.
