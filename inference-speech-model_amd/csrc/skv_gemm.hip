@@ -314,10 +314,8 @@ int skv_rows_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
   float us = 0.f;
   const int tile = pick_tile(p.m, p.n, (int)cdiv(kb, kBk), act != 0, &us);
   // own / library measured (us, bf16, GELU): 130 x 5120 x 1280 10.1 / 14.4, 512 x 2048 x 512 7.4 / 12.1, 1500 x 5120 x 1280
-  // 30.1 / 31.9 (estimates' ratio 0.89), 400 x 5120 x 1280 18.9 / 19.3 (0.94); the library: 3000 x 4096 x 1024 44.7 / 38.4
-  // (0.99), 1608 x 5120 x 1280 38.7 / 34.2 (1.05), 3000 x 5120 x 1280 59.7 / 48.3. The library's line is that of one version;
-  // with another both ways stay right and the crossover may lie elsewhere.
-  if (act && us > 0.98f * library_gelu_us((float)m, (float)n, (float)k))
+  // 31.4 / 33.9, 6000 x 3072 x 768 51 / 71; the library: 1608 x 5120 x 1280 38.7 / 36.1, 3000 x 5120 x 1280 59.7 / 54.1.
+  if (act && us > 1.05f * library_gelu_us((float)m, (float)n, (float)k))
     return fail(SKV_EUNSUPPORTED, "%s: m=%d n=%d k=%d fills the units badly", who, m, n, k);
   p.tiles_m = (uint32_t)cdiv(m, 64 * kTiles[tile].mi);
   p.tiles_n = (uint32_t)cdiv(n, 64 * kTiles[tile].ni);
