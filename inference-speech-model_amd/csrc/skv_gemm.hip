@@ -227,7 +227,8 @@ constexpr Tile kTiles[] = {{1, 1, 0.256f}, {1, 2, 0.328f}, {2, 1, 0.334f}, {2, 2
 // The tile with the least estimated time, and that time (us). A unit's workgroups share it, so the steps and epilogues of
 // all of them add up (up to 128 x 128 two are resident; the largest tiles' run one after the other); past two rounds
 // the last one is half empty on average. Estimate / measured (bf16): 1500 x 5120 x 1280 128 x 128 26.4 / 26.5, 192 x 128
-// 38.4 / 38.1; 512 x 1280 x 1280 64 x 64 9.1 / 9.1; 1500 x 3840 x 1280 192 x 128 19.2 / 21.9, 128 x 128 26.5 / 23.8.
+// 41.4 / 38.1; 512 x 1280 x 1280 64 x 64 9.1 / 9.1; 1500 x 3840 x 1280 192 x 128 20.7 / 21.9, 128 x 128 26.5 / 23.8; with
+// GELU 3000 x 4096 x 1024 192 x 128 44.6 / 44.7 (the library and its GELU launch 38.4).
 int pick_tile(uint32_t m, uint32_t n, int steps, bool act, float* us) {
   int best = 0;
   float best_cost = 1e30f;
@@ -237,7 +238,7 @@ int pick_tile(uint32_t m, uint32_t n, int steps, bool act, float* us) {
     const int64_t tiles = cdiv(m, 64 * t.mi) * cdiv(n, 64 * t.ni);
     const float rounds = tiles > 2 * cus ? (float)tiles / (float)cus + 0.5f : (float)cdiv(tiles, cus);
     const float area = (float)(t.mi * t.ni);
-    const float cost = rounds * ((float)steps * t.step + (act ? 1.37f : 0.72f) * area) + 3.3f * (area > 4.f ? rounds : 1.f);
+    const float cost = rounds * ((float)steps * t.step + (act ? 1.37f : 0.72f) * area) + (area > 4.f ? 4.8f * rounds : 3.3f);
     if (cost < best_cost) best = i, best_cost = cost;
   }
   *us = best_cost;
@@ -314,7 +315,9 @@ int skv_rows_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
   float us = 0.f;
   const int tile = pick_tile(p.m, p.n, (int)cdiv(kb, kBk), act != 0, &us);
   // own / library measured (us, bf16, GELU): 130 x 5120 x 1280 10.1 / 14.4, 512 x 2048 x 512 7.4 / 12.1, 1500 x 5120 x 1280
-  // 31.4 / 33.9, 6000 x 3072 x 768 51 / 71; the library: 1608 x 5120 x 1280 38.7 / 36.1, 3000 x 5120 x 1280 59.7 / 54.1.
+  // 30.1 / 31.9, 1608 x 4096 x 1024 25.2 / 27.9; the library: 3000 x 4096 x 1024 44.7 / 38.4, 1608 x 5120 x 1280 38.7 / 34.2,
+  // 3000 x 5120 x 1280 59.7 / 48.3. The library's line is that of one version: with another both ways stay right, and the
+  // crossover may lie elsewhere.
   if (act && us > 1.05f * library_gelu_us((float)m, (float)n, (float)k))
     return fail(SKV_EUNSUPPORTED, "%s: m=%d n=%d k=%d fills the units badly", who, m, n, k);
   p.tiles_m = (uint32_t)cdiv(m, 64 * kTiles[tile].mi);
