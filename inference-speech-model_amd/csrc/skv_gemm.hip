@@ -5,7 +5,8 @@
 // L1 at the 31-50 bytes a clock that its 32 KB of lines in flight allow). Hence 128 x 128 and smaller tiles with
 // 32 x 32 x 16 products, rows two steps ahead in registers (one step: 1500 x 1280 x 5120 64 us, two: 39), LDS rows
 // swizzled instead of padded (padded: 260 of 1050 LDS clocks a step were conflicts), and LDS operations placed between
-// products. What the library's GEMM cannot do is in the epilogue: GELU on the fp32 sums, and K and V written by head.
+// products. What the library's GEMM cannot do is in the epilogue: GELU on the fp32 sums, and K and V written by head (and
+// a residual add, for callers of the C interface: the models' adds share the LayerNorm's launch).
 // Measured (us, bf16, against the library's GEMM and the launches it needs): q/k/v 1500 x 3840 x 1280 with K and V by head
 // 24 / 32, 512 x 1152 x 384 5.4 / 14.6, 12000 x 2304 x 768 59 / 93; with GELU 1500 x 5120 x 1280 32 / 34,
 // 512 x 2048 x 512 7.3 / 12.1, 130 x 5120 x 1280 10.3 / 14.5.
