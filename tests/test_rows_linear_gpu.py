@@ -1,7 +1,7 @@
 """Projections of many rows (skv_rows_linear) against float64: bias, GELU, residual, and q/k/v columns by head.
 
-Sizes sit at the edges of the kernel's 64- to 192-row tiles and 128-byte steps; the last four take each of its larger
-tiles. The bar is the output's rounding plus the fp32 accumulation bound k * 2^-24 * sum |x w|.
+Sizes sit at the edges of the kernel's 64- to 192-row tiles and 128-byte steps; the last four of SIZES and the two of
+MORE_TILES take its larger tiles. The bar is the output's rounding plus the fp32 accumulation bound k * 2^-24 * sum |x w|.
 """
 import pytest
 import torch
@@ -14,6 +14,8 @@ pytestmark = pytest.mark.gpu
 EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
 SIZES = [(1, 8, 8), (63, 64, 64), (64, 72, 72), (65, 128, 136), (129, 200, 1288), (300, 1288, 200), (1000, 136, 2056),
          (1500, 1280, 1280), (1500, 3840, 1288), (1500, 5120, 1280), (1300, 8200, 640)]
+
+MORE_TILES = [(1801, 1072, 328), (1751, 3272, 328)]  # 128 x 64 and 128 x 192 outputs, the last tiles nearly empty
 
 
 def _data(m, n, k, dt):
@@ -77,3 +79,12 @@ def test_strides_and_refused_calls(cuda):
     assert torch.allclose(y.double(), F.gelu(ref + b.double()), rtol=1e-3, atol=1e-3)
     x[77, 3] = float("nan")  # reaches its own row only
     assert torch.isnan(native.rows_linear(x, w)).any(dim=1).nonzero().flatten().tolist() == [77]
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("size", MORE_TILES)
+def test_rows_linear_over_the_other_tiles(cuda, dt, size):
+    x, w, b, r, ref, bound = _data(*size, dt)
+    few = 2.0 ** -21 * (ref.abs() + b.double().abs() + r.double().abs())
+    _check(native.rows_linear(x, w), ref, bound, "plain")
+    _check(native.rows_linear(x, w, b, res=r), ref + b.double() + r.double(), bound + few, "bias, residual")
