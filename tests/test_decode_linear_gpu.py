@@ -201,3 +201,27 @@ def test_normed_projection_is_as_exact_as_the_layernorm_launch(cuda, dt):
         n = native.add_layernorm(s, None, one, zeros.new_zeros(d), 1e-5)[1]
         err, ref = (float((t.double() - want).norm()) for t in (y, n))
         assert err <= (1.1 if dt == torch.float32 else 1.01) * ref, (mean, d, err, ref)
+
+
+# 31 x 2052 and 31 x 4100 outputs take tiles of 32 x 16 and 32 x 32, 64 x 4100 of 64 x 32; k (16-bit) one length for each of the
+# kernel's wave and round counts, with a partial last chunk or round where there is room for one
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k16", [256, 480, 768, 992, 1280, 2048])
+def test_every_tile_plain_and_normed(cuda, dt, k16):
+    k = k16 if dt != torch.float32 else k16 // 2
+    g = torch.Generator(device="cuda").manual_seed(k16)
+    zeros = torch.zeros(64, 256, device="cuda", dtype=dt)
+    gm, bt = (torch.randn(k, generator=g, device="cuda").to(dt) for _ in range(2))
+    for m, n in ((16, 20), (31, 2052), (31, 4100), (64, 4100)):
+        x, w, b, ref, bound = _data(m, n, k, dt, m + n)
+        _check(native.decode_linear(x, w, b), ref, bound, f"m={m} n={n} k={k}")
+        s, stats = native.decode_linear_residual(zeros[:m], zeros.new_zeros(k, 256), None, x)
+        assert torch.equal(s, x)
+        y = native.decode_linear_normed(s, stats, gm, bt, 1e-5, w, b)
+        assert (y is None) == (m == 64)  # tiles of 64 rows leave the LayerNorm to a launch
+        if y is not None:
+            want = F.layer_norm(s.double(), (k,), gm.double(), bt.double(), 1e-5)
+            # each normalised element rounded to dtype (and a few fp32 roundings), then the product's own bound
+            slack = (2 * EPS[dt] + (k + 8) * 2.0 ** -24) * (want.abs() + 1e-2) @ w.double().abs().t() + 1e-6
+            ref = want @ w.double().t() + b.double()
+            _check(y, ref, slack + 2.0 ** -20 * ref.abs(), f"normed m={m} n={n} k={k}")
